@@ -432,8 +432,8 @@ def set_tune(dtype="float64", **fields):
     """Change the global launch setting (unspecified fields keep their
     value): ``diag_max_l``, ``adj_wg``, ``order``, ``fuse_max_n``,
     ``adj_algo`` (0 = adjoint over 8x8x8 tiles, the default; 1 = node by
-    node) and ``fwd_segs`` (c segments of the diagonal forward, 1..8; 0 =
-    8)."""
+    node) and ``fwd_segs`` (c segments of the diagonal forward, 1..8; 0, the
+    default: the library chooses, 8 segments or several workgroups per event)."""
     t = L.AdtTune()
     L.check(L.lib().adt_get_tune(_dtype_code(dtype), ctypes.byref(t)), "get_tune")
     _apply(t, fields)

@@ -12,6 +12,7 @@
 #include <list>
 #include <map>
 #include <mutex>
+#include <set>
 #include <string>
 #include <type_traits>
 #include <utility>
@@ -106,6 +107,10 @@ ClassKey class_of(int64_t m, int64_t n, int64_t l) {
   return k;
 }
 std::map<ClassKey, adt_tune> g_classes[2];
+// Classes whose events the autotuner found faster with several workgroups
+// each: their setting's fwd_segs then holds for launches that do not take that
+// path.  Setting a class by hand fixes its kernel.
+std::set<ClassKey> g_open[2];
 
 template <typename T>
 constexpr int tune_index() {
@@ -115,6 +120,11 @@ constexpr int tune_index() {
 struct TuneSnap {
   adt_tune global;
   std::map<ClassKey, adt_tune> classes;
+  std::set<ClassKey> open;
+  // may the library choose the forward kernel of an event of this box?
+  bool leaves_open(int64_t m, int64_t n, int64_t l) const {
+    return for_box(m, n, l).fwd_segs == 0 || open.count(class_of(m, n, l)) > 0;
+  }
   // the setting of an event of box (m, n, l): its class's per-event fields
   // over the global setting
   adt_tune for_box(int64_t m, int64_t n, int64_t l) const {
@@ -131,7 +141,7 @@ struct TuneSnap {
 template <typename T>
 TuneSnap current_snap() {
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  return TuneSnap{g_tune[tune_index<T>()], g_classes[tune_index<T>()]};
+  return TuneSnap{g_tune[tune_index<T>()], g_classes[tune_index<T>()], g_open[tune_index<T>()]};
 }
 template <typename T>
 adt_tune current_tune() {
@@ -151,12 +161,13 @@ bool tune_valid(const adt_tune& t) {
 const char* const kTuneFields[] = {"diag_max_l", "adj_wg", "order", "fuse_max_n",
                                    "fwd_ms", "adj_ms", "adj_algo", "fwd_segs"};
 
-std::string tune_json(int dtype, const adt_tune& t, const ClassKey* k) {
+std::string tune_json(int dtype, const adt_tune& t, const ClassKey* k, bool open = false) {
   char buf[512];
   int o = snprintf(buf, sizeof buf, "{\"dtype\": %d, ", dtype);
   if (k)
     o += snprintf(buf + o, sizeof buf - o, "\"l_blocks\": %d, \"bands\": %d, \"log2n\": %d, ",
                   k->l_blocks, k->bands, k->log2n);
+  if (open) o += snprintf(buf + o, sizeof buf - o, "\"open\": 1, ");
   snprintf(buf + o, sizeof buf - o,
            "\"diag_max_l\": %d, \"adj_wg\": %d, \"order\": %d, \"fuse_max_n\": %d, "
            "\"fwd_ms\": %.9g, \"adj_ms\": %.9g, \"adj_algo\": %d, \"fwd_segs\": %d}",
@@ -168,7 +179,7 @@ std::string tune_json(int dtype, const adt_tune& t, const ClassKey* k) {
 // Reads the objects of the text written by tune_json (keys in any order,
 // numbers only); every field must be present.
 int parse_tune_json(const std::string& txt, adt_tune glob[2], bool have_glob[2],
-                    std::map<ClassKey, adt_tune> cls[2]) {
+                    std::map<ClassKey, adt_tune> cls[2], std::set<ClassKey> open[2]) {
   size_t i = 0;
   std::string section;
   while (i < txt.size()) {
@@ -223,6 +234,8 @@ int parse_tune_json(const std::string& txt, adt_tune glob[2], bool have_glob[2],
       if (!get("l_blocks", &lb) || !get("bands", &bd) || !get("log2n", &lg))
         return fail(ADT_EINVAL, "tune file: class without l_blocks / bands / log2n");
       cls[di][ClassKey{(int)lb, (int)bd, (int)lg}] = t;
+      double op = 0;  // (files of before this key: off)
+      if (get("open", &op) && op == 1) open[di].insert(ClassKey{(int)lb, (int)bd, (int)lg});
     }
   }
   return ADT_OK;
@@ -360,6 +373,106 @@ void set_event_setting(adt::EventDesc& d, const adt_tune& t) {
   d.adj_algo = (int8_t)adj_algo_for(t.adj_algo, tiles_of(d.m, d.n, d.l));
 }
 
+// ---- several workgroups per event (fwd3_team_kernel)
+
+// The library's choice of forward kernel for a set of events whose setting
+// leaves it open (diagonal forward, fwd_segs 0).
+int device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 256;
+  return n > 0 ? n : 256;
+}
+
+struct TeamPlan {
+  std::vector<adt::TeamDesc> descs;  // words: byte offsets until bind()
+  size_t off_desc = 0, off_zero = 0, zero_bytes = 0;
+  int per_group = 1, grid = 0;
+  bool on() const { return !descs.empty(); }
+
+  template <typename T>
+  static bool fits(const adt::EventDesc& d) {
+    const double big = sizeof(T) == 8 ? 0x1p240 : 0x1p20;
+    return d.fwd_diag && std::fabs(d.h) < big &&
+           std::max(d.m, d.n) < (1 << adt::kTeamSeqShift) - 64;
+  }
+  template <typename T>
+  static adt::TeamDesc geometry(const adt::EventDesc& d) {
+    const int64_t LW = 16 / (int64_t)sizeof(T);
+    adt::TeamDesc t{};
+    const int Ma = std::min(d.m, d.n);
+    t.bands = (Ma + 63) / 64;
+    t.H = (Ma + t.bands - 1) / t.bands;
+    t.bands = (Ma + t.H - 1) / t.H;
+    t.ns = (int)((d.l + LW * adt::kTW - 1) / (LW * adt::kTW));
+    t.R = t.bands * t.ns;
+    const int64_t N = (int64_t)d.m * d.n * d.l;
+    t.E = (int)std::max<int64_t>(1, std::min<int64_t>(32, N / 8192));
+    return t;
+  }
+  // Lays out the words of the events `use` (indices into evs) from byte
+  // offset `off` on; returns the end.
+  template <typename T>
+  size_t build(std::vector<adt::EventDesc>& evs, const std::vector<int>& use, size_t off) {
+    auto take = [&](size_t b) {
+      const size_t o = off;
+      off += ((b + 255) / 256) * 256;
+      return o;
+    };
+    const int nt = (int)use.size();
+    descs.clear();
+    off_desc = take(sizeof(adt::TeamDesc) * nt);
+    off_zero = take(sizeof(adt::TeamShared) + sizeof(int) * (size_t)adt::kTeamXcds * nt);
+    int64_t maxR = 1;
+    for (int e : use) {
+      adt::TeamDesc t = geometry<T>(evs[e]);
+      t.ev = e;
+      t.words = (int*)take(sizeof(int) * adt::team_words(t.R));
+      evs[e].team_words = t.words;
+      maxR = std::max<int64_t>(maxR, t.R);
+      descs.push_back(t);
+    }
+    zero_bytes = off - off_zero;
+    // workgroups: up to 4 per compute unit (the kernel's occupancy); an event
+    // has work for about 2.5 sweeps' regions at a time
+    const int cus = device_cus(), xcds = std::max(1, cus / 32);
+    const int slots = 4 * cus / xcds;
+    const int here = (nt + xcds - 1) / xcds;  // events per XCD at a time
+    per_group = (int)std::max<int64_t>(1, std::min<int64_t>(slots / std::min(here, slots),
+                                                          (5 * maxR + 1) / 2 + 1));
+    grid = xcds * std::min(slots, here * per_group);
+    return off;
+  }
+  void bind(char* base, std::vector<adt::EventDesc>& evs) {
+    for (auto& t : descs) {
+      t.words = (int*)(base + (size_t)t.words);
+      evs[t.ev].team_words = t.words;
+    }
+  }
+  template <typename T>
+  void launch(bool mix, const adt::EventDesc* d, char* base, hipStream_t s) const {
+    const adt::TeamDesc* td = (const adt::TeamDesc*)(base + off_desc);
+    adt::TeamShared* sh = (adt::TeamShared*)(base + off_zero);
+    const int nt = (int)descs.size();
+    if constexpr (std::is_same<T, float>::value) {
+      if (mix) {
+        adt::fwd3_team_kernel<float, true>
+            <<<grid, adt::kTW * 64, 0, s>>>(d, td, sh, nt, per_group, kMaxIter3);
+        return;
+      }
+    }
+    adt::fwd3_team_kernel<T, false>
+        <<<grid, adt::kTW * 64, 0, s>>>(d, td, sh, nt, per_group, kMaxIter3);
+  }
+};
+
+void launch_clear(adt_info* infos, int nev, void* words, size_t bytes, hipStream_t s) {
+  const size_t nw = bytes / sizeof(int);
+  const int grid = (int)std::max<size_t>(1, std::min<size_t>(256, (nw + 1023) / 1024));
+  adt::info_clear_kernel<<<grid, 256, 0, s>>>(infos, nev, (int*)words, (int64_t)nw);
+}
+
 template <typename T>
 int fwd3_impl(const T* u0, const T* f, T h, int64_t m, int64_t n, int64_t l, T tol, int verbose,
               T* u, adt_info* info, int flags, void* stream) {
@@ -377,12 +490,11 @@ int fwd3_impl(const T* u0, const T* f, T h, int64_t m, int64_t n, int64_t l, T t
   if ((rc = st.in(u0, bytes, hp, &du0, s)) || (rc = st.in(f, bytes, hp, &df, s)) ||
       (rc = st.out(u, bytes, hp, &du, s)))
     return rc;
-  DevBuf ws;
-  const size_t off_desc = ((bytes + 255) / 256) * 256;
-  const size_t off_info = off_desc + 256;
-  if ((rc = ws.alloc(off_info + sizeof(adt_info), s))) return rc;
-  char* base = (char*)ws.p;
-  adt::EventDesc d{};
+  const TuneSnap snap = current_snap<T>();
+  const adt_tune tn = snap.for_box(m, n, l);
+  std::vector<adt::EventDesc> ds(1);
+  adt::EventDesc& d = ds[0];
+  d = adt::EventDesc{};
   d.m = (int)m;
   d.n = (int)n;
   d.l = (int)l;
@@ -391,16 +503,34 @@ int fwd3_impl(const T* u0, const T* f, T h, int64_t m, int64_t n, int64_t l, T t
   d.u0 = du0;
   d.f = df;
   d.u = du;
+  set_event_setting(d, tn);
+  // one event leaves all other compute units idle: several workgroups for it
+  TeamPlan team;
+  const size_t off_info = ((bytes + 255) / 256) * 256;
+  const size_t off_desc = off_info + ((sizeof(adt_info) + 255) / 256) * 256;
+  size_t end = off_desc + 256;
+  if (snap.leaves_open(m, n, l) && TeamPlan::fits<T>(d)) end = team.build<T>(ds, {0}, end);
+  DevBuf ws;
+  if ((rc = ws.alloc(end, s))) return rc;
+  char* base = (char*)ws.p;
   d.uold = base;
   d.info = (adt_info*)(base + off_info);
-  set_event_setting(d, current_snap<T>().for_box(m, n, l));
-  ADT_HIP(hipMemcpyAsync(base + off_desc, &d, sizeof(d), hipMemcpyHostToDevice, s));
-  adt::info_clear_kernel<<<1, 64, 0, s>>>(d.info, 1);
+  team.bind(base, ds);
+  // the two descriptors in one copy
+  char hdesc[512];
+  static_assert(sizeof(adt::EventDesc) <= 256 && sizeof(adt::TeamDesc) <= 256, "descriptor slots");
+  memcpy(hdesc, &d, sizeof(d));
+  if (team.on()) memcpy(hdesc + 256, &team.descs[0], sizeof(adt::TeamDesc));
+  ADT_HIP(hipMemcpyAsync(base + off_desc, hdesc, team.on() ? 256 + sizeof(adt::TeamDesc) : sizeof(d),
+                         hipMemcpyHostToDevice, s));
+  const adt::EventDesc* dd = (const adt::EventDesc*)(base + off_desc);
+  launch_clear(d.info, 1, base + team.off_zero, team.zero_bytes, s);
   const bool mix = flags & ADT_F32_COMPUTE_F64;
+  if (team.on()) team.launch<T>(mix, dd, base, s);
   if (d.fwd_diag)
-    launch_fwd_diag<T>(mix, 1, (const adt::EventDesc*)(base + off_desc), s);
+    launch_fwd_diag<T>(mix, 1, dd, s);
   else
-    launch_fwd_stream<T>(mix, 1, (const adt::EventDesc*)(base + off_desc), s);
+    launch_fwd_stream<T>(mix, 1, dd, s);
   ADT_HIP(hipGetLastError());
   adt_info hinf{};
   ADT_HIP(hipMemcpyAsync(&hinf, d.info, sizeof(adt_info), hipMemcpyDeviceToHost, s));
@@ -478,7 +608,7 @@ int fwd3_noalloc_impl(const double* u0, const double* f, double h, int64_t m, in
   d.info = (adt_info*)(b + kNoAllocInfoOff);
   set_event_setting(d, current_snap<double>().for_box(m, n, l));
   ADT_HIP(hipMemcpyAsync(b + kNoAllocDescOff, &d, sizeof(d), hipMemcpyHostToDevice, s));
-  adt::info_clear_kernel<<<1, 64, 0, s>>>(d.info, 1);
+  launch_clear(d.info, 1, nullptr, 0, s);
   if (d.fwd_diag)
     launch_fwd_diag<double>(false, 1, (const adt::EventDesc*)(b + kNoAllocDescOff), s);
   else
@@ -543,7 +673,7 @@ int bwd3_impl(const T* g, const T* u, const T* u0, const T* f, T h, int64_t m, i
   const size_t od = a + c + q;
   d.info = (adt_info*)(base + od + 256);
   ADT_HIP(hipMemcpyAsync(base + od, &d, sizeof(d), hipMemcpyHostToDevice, s));
-  adt::info_clear_kernel<<<1, 64, 0, s>>>(d.info, 1);
+  launch_clear(d.info, 1, nullptr, 0, s);
   launch_adj<T>(algo, tiles, 1, (const adt::EventDesc*)(base + od), tn.adj_wg, s);
   ADT_HIP(hipGetLastError());
   adt_info hinf{};
@@ -592,7 +722,7 @@ int fwd2_impl(const T* f, int64_t m, int64_t n, int64_t srcx, int64_t srcy, T h,
   d.uold = base;
   d.info = (adt_info*)(base + a + 256);
   ADT_HIP(hipMemcpyAsync(base + a, &d, sizeof(d), hipMemcpyHostToDevice, s));
-  adt::info_clear_kernel<<<1, 64, 0, s>>>(d.info, 1);
+  launch_clear(d.info, 1, nullptr, 0, s);
   adt::fwd2_event_kernel<T><<<1, kWG, 0, s>>>((const adt::Event2Desc*)(base + a), kMaxIter2);
   ADT_HIP(hipGetLastError());
   adt_info hinf{};
@@ -643,7 +773,7 @@ int bwd2_impl(const T* g, const T* u, const T* f, int64_t m, int64_t n, int64_t 
   const size_t od = a + 2 * c + q;
   d.info = (adt_info*)(base + od + 256);
   ADT_HIP(hipMemcpyAsync(base + od, &d, sizeof(d), hipMemcpyHostToDevice, s));
-  adt::info_clear_kernel<<<1, 64, 0, s>>>(d.info, 1);
+  launch_clear(d.info, 1, nullptr, 0, s);
   adt::adj2_kahn_kernel<T><<<1, kWG, 0, s>>>((const adt::Event2Desc*)(base + od));
   ADT_HIP(hipGetLastError());
   adt_info hinf{};
@@ -1003,6 +1133,44 @@ struct KernelMix {
   int64_t max_n = 0;     // largest node count
 };
 
+// Forward and adjoint of each event in one kernel: every event on the
+// diagonal forward and the node-level adjoint.
+bool fused(int flags, const KernelMix& km, const adt_tune& tn) {
+  return (flags & ADT_FORWARD) && (flags & ADT_ADJOINT) && km.diag && !km.stream && km.node &&
+         !km.tile && km.max_n <= tn.fuse_max_n;
+}
+
+// Do several workgroups per event pay for these events?  Both kernels' times
+// for one iteration, from the steps they take (microseconds a step as measured
+// on an MI355X; the iteration counts are the same):
+//   one workgroup per event: bands * N_b + H + 6 steps per sweep and k chunk,
+//     2.4 us + 0.27 us per node of a lane, events in parallel over the CUs;
+//   team: an event alone takes 4 (M_a + N_b) + 30 slabs + 80 steps (its sweeps
+//     overlap) of 1.1 us; many events are bound by their 16-byte accesses to
+//     the L2, 0.44 us per CU for each wave step.
+// 256 events of 128x128x64 FP64: 37 ms against 130 ms; 64 with FP32 storage: 28
+// against 18 ms; one: 28 against 5.5 ms.
+template <typename T>
+bool team_pays(const std::vector<adt::EventDesc>& descs) {
+  const double cus = device_cus();
+  double dmax = 0, dsum = 0, tmax = 0, tsum = 0;
+  for (const adt::EventDesc& d : descs) {
+    const adt::TeamDesc t = TeamPlan::geometry<T>(d);
+    const double Ma = std::min(d.m, d.n), Nb = std::max(d.m, d.n);
+    double one = 0;
+    for (int c = 0; c < d.l; c += 8 * kSegsMax) {
+      const int lw = (std::min(d.l - c, 8 * kSegsMax) + kSegsMax - 1) / kSegsMax;
+      one += 8 * (t.bands * Nb + t.H + 6) * (2.4 + 0.27 * lw);
+    }
+    const double segs = (d.l * (double)sizeof(T) + 15) / 16;
+    dmax = std::max(dmax, one);
+    dsum += one;
+    tmax = std::max(tmax, (4 * (Ma + Nb) + 30 * t.ns + 80) * 1.1);
+    tsum += 8 * t.bands * (Nb + t.H - 1) * segs * 0.44;
+  }
+  return std::max(tmax, tsum / cus) < 0.9 * std::max(dmax, dsum / cus);
+}
+
 template <typename T>
 struct BatchPlan {
   std::vector<adt::EventDesc> descs;
@@ -1014,6 +1182,7 @@ struct BatchPlan {
   const MisfitArgs* mis = nullptr;
   size_t off_mis = 0, off_coords = 0;
   RecvNodes<T> rnodes;
+  TeamPlan team;  // events with several workgroups each
 
   // Each event's receiver misfit runs between its forward and its adjoint
   // and writes its grad_u: the item must name the event's u and grad_u.
@@ -1055,6 +1224,13 @@ struct BatchPlan {
       descs[e].mnodes = (const adt::MisfitNodes*)(rnodes.o_tab + sizeof(adt::MisfitNodes) * e);
       descs[e].nrec = m->nrec;
     }
+    return ADT_OK;
+  }
+  // Device copy of the team descriptors (after bind()).
+  int upload_teams(char* base, hipStream_t s) {
+    if (team.on())
+      ADT_HIP(hipMemcpyAsync(base + team.off_desc, team.descs.data(),
+                             sizeof(adt::TeamDesc) * team.descs.size(), hipMemcpyHostToDevice, s));
     return ADT_OK;
   }
   // Device copies of the misfit table and coordinates (after bind()).
@@ -1107,6 +1283,7 @@ struct BatchPlan {
       descs[e].fwd_diag = x.l <= t.diag_max_l ? 1 : 0;
       descs[e].fwd_segs = (int8_t)(t.fwd_segs > 0 ? t.fwd_segs : kSegsMax);
       descs[e].adj_algo = (int8_t)adj_algo_for(t.adj_algo, tiles);
+      descs[e].pad = snap.leaves_open(x.m, x.n, x.l) ? 1 : 0;
       if (flags & ADT_FORWARD) (descs[e].fwd_diag ? mix.diag : mix.stream) = true;
       if (flags & ADT_ADJOINT) {
         if (descs[e].adj_algo == 0) {
@@ -1160,7 +1337,22 @@ struct BatchPlan {
       return (int64_t)a.m * a.n * a.l > (int64_t)b.m * b.n * b.l;
     });
   }
+  // Routes the forward to fwd3_team_kernel where the settings leave the
+  // choice open and the events are too few or too uneven for one workgroup
+  // each; after order_largest_first (the plan's indices are final).
+  void plan_teams(int flags, const adt_tune& tn) {
+    if (!(flags & ADT_FORWARD) || descs.empty()) return;
+    if (fused(flags, mix, tn)) return;
+    std::vector<int> use;
+    for (size_t e = 0; e < descs.size(); ++e) {
+      if (!descs[e].pad || !TeamPlan::fits<T>(descs[e])) return;
+      use.push_back((int)e);
+    }
+    if (!team_pays<T>(descs)) return;
+    ws_bytes = team.build<T>(descs, use, ws_bytes);
+  }
   void bind(char* base) {
+    team.bind(base, descs);
     for (auto& d : descs) {
       d.uold = base + (size_t)d.uold;
       d.lam = base + (size_t)d.lam;
@@ -1184,17 +1376,18 @@ struct BatchPlan {
 // names (each kernel skips the other's events), the misfit, then each
 // event's adjoint traversal likewise.  tn: the launch-wide fields.
 template <typename T>
-int launch_batch(const adt::EventDesc* ddesc, int nev, int flags, const KernelMix& km,
-                 const adt_tune& tn, adt_info* infos, hipStream_t s,
-                 const MisfitRun& mr = MisfitRun{}) {
+int launch_batch(const BatchPlan<T>& plan, char* base, int nev, int flags, const adt_tune& tn,
+                 hipStream_t s, const MisfitRun& mr = MisfitRun{}) {
   if (nev == 0) return ADT_OK;
-  adt::info_clear_kernel<<<1, 256, 0, s>>>(infos, nev);
+  const adt::EventDesc* ddesc = (const adt::EventDesc*)(base + plan.off_desc);
+  const KernelMix& km = plan.mix;
+  const TeamPlan& team = plan.team;
+  launch_clear((adt_info*)(base + plan.off_info), nev, base + team.off_zero, team.zero_bytes, s);
   ADT_HIP(hipGetLastError());
   const bool mix = flags & ADT_F32_COMPUTE_F64;
   // forward and adjoint of each event in one kernel (every event on the
   // diagonal forward and the node-level adjoint)
-  if ((flags & ADT_FORWARD) && (flags & ADT_ADJOINT) && km.diag && !km.stream && km.node &&
-      !km.tile && km.max_n <= tn.fuse_max_n) {
+  if (fused(flags, km, tn)) {
     if constexpr (std::is_same<T, float>::value) {
       if (mix) {
         adt::fwd_adj3_diag_kernel<float, true><<<nev, kDiagWG, 0, s>>>(ddesc, kMaxIter3);
@@ -1207,7 +1400,11 @@ int launch_batch(const adt::EventDesc* ddesc, int nev, int flags, const KernelMi
     return ADT_OK;
   }
   if (flags & ADT_FORWARD) {
-    if (km.diag) {
+    if (team.on()) {
+      team.launch<T>(mix, ddesc, base, s);
+      ADT_HIP(hipGetLastError());
+    }
+    if (km.diag) {  // after the team kernel: only the events that it left
       launch_fwd_diag<T>(mix, nev, ddesc, s);
       ADT_HIP(hipGetLastError());
     }
@@ -1249,16 +1446,16 @@ int batched_impl(const adt_event3d* ev, int nev, int flags, adt_info* infos, voi
   if (mis && (rc = plan.attach_misfit(ev, nev, mis))) return rc;
   if (nev == 0) return ADT_OK;
   if (tn.order) plan.order_largest_first();
+  plan.plan_teams(flags, tn);
   DevBuf ws;
   if ((rc = ws.alloc(plan.ws_bytes, s))) return rc;
   plan.bind((char*)ws.p);
   char* base = (char*)ws.p;
   ADT_HIP(hipMemcpyAsync(base + plan.off_desc, plan.descs.data(), sizeof(adt::EventDesc) * nev,
                          hipMemcpyHostToDevice, s));
+  if ((rc = plan.upload_teams(base, s))) return rc;
   if ((rc = plan.upload_misfit(base, nev, s))) return rc;
-  if ((rc = launch_batch<T>((const adt::EventDesc*)(base + plan.off_desc), nev, flags, plan.mix,
-                            tn, (adt_info*)(base + plan.off_info), s, plan.misfit_run(base))))
-    return rc;
+  if ((rc = launch_batch<T>(plan, base, nev, flags, tn, s, plan.misfit_run(base)))) return rc;
   // the misfit table and coordinates were copied from the caller's host
   // memory: wait before returning
   if (mis && !infos) ADT_HIP(hipStreamSynchronize(s));
@@ -1400,8 +1597,8 @@ int bwd3_plain_impl(const T* g, const T* u, const T* u0, const T* f, T h, int64_
 
 // Times launch settings on the caller's events and keeps the fastest.
 // First, for each box-shape class among the events and on that class's
-// events alone: the forward kernel (k-streaming, or diagonal streaming with
-// 8, 4 or ceil(l / 8) c segments) and then the adjoint traversal (tiles or
+// events alone: the forward kernel (k-streaming, diagonal streaming with
+// 8, 4 or ceil(l / 8) c segments, or several workgroups per event) and then the adjoint traversal (tiles or
 // node by node), stored as the class's setting.  Then, on all events with
 // those class settings: the event order, the node-level adjoint's
 // workgroup size, and whether the fused forward + adjoint kernel beats the
@@ -1443,18 +1640,18 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
     int r = plan.build(evs.data(), n, fl, sn);
     if (r) return r;
     if (sn.global.order) plan.order_largest_first();
+    plan.plan_teams(fl, sn.global);
     DevBuf ws;
     if ((r = ws.alloc(plan.ws_bytes, s))) return r;
     plan.bind((char*)ws.p);
     char* base = (char*)ws.p;
-    const adt::EventDesc* dd = (const adt::EventDesc*)(base + plan.off_desc);
-    adt_info* inf = (adt_info*)(base + plan.off_info);
     ADT_HIP(hipMemcpyAsync(base + plan.off_desc, plan.descs.data(), sizeof(adt::EventDesc) * n,
                            hipMemcpyHostToDevice, s));
-    if ((r = launch_batch<T>(dd, n, fl, plan.mix, sn.global, inf, s))) return r;
+    if ((r = plan.upload_teams(base, s))) return r;
+    if ((r = launch_batch<T>(plan, base, n, fl, sn.global, s))) return r;
     ADT_HIP(hipEventRecord(e0, s));
     for (int k = 0; k < reps; ++k)
-      if ((r = launch_batch<T>(dd, n, fl, plan.mix, sn.global, inf, s))) return r;
+      if ((r = launch_batch<T>(plan, base, n, fl, sn.global, s))) return r;
     ADT_HIP(hipEventRecord(e1, s));
     ADT_HIP(hipEventSynchronize(e1));
     ADT_HIP(hipEventElapsedTime(ms, e0, e1));
@@ -1462,7 +1659,25 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
     return ADT_OK;
   };
   int rc = ADT_OK;
+  // several workgroups per event (fwd_segs 0) where that is the library's
+  // choice for all of the events
+  bool team_ok = false;
+  if (flags & ADT_FORWARD) {
+    std::vector<adt::EventDesc> ds(nev);
+    team_ok = true;
+    for (int e = 0; e < nev; ++e) {
+      ds[e] = adt::EventDesc{};
+      ds[e].m = (int)ev[e].m;
+      ds[e].n = (int)ev[e].n;
+      ds[e].l = (int)ev[e].l;
+      ds[e].h = ev[e].h;
+      ds[e].fwd_diag = 1;
+      team_ok = team_ok && TeamPlan::fits<T>(ds[e]);
+    }
+    team_ok = team_ok && team_pays<T>(ds);
+  }
   std::map<ClassKey, adt_tune> classes = cur.classes;
+  std::set<ClassKey> open = cur.open;
   // --- per class: forward kernel and segments, then adjoint traversal
   for (auto it = groups.begin(); it != groups.end() && rc == ADT_OK; ++it) {
     const std::vector<adt_event3d>& evs = it->second;
@@ -1499,6 +1714,20 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
         }
       }
       if (rc) break;
+      open.erase(it->first);
+      if (team_ok) {
+        TuneSnap t1 = sc;
+        t1.classes.clear();
+        t1.open.clear();
+        t1.global.diag_max_l = adt::kDiagAll;
+        t1.global.fwd_segs = 0;
+        float ms = 0.f;
+        if ((rc = time_set(evs, t1, ADT_FORWARD | fmix, &ms))) break;
+        if (ms < fbest && sc.global.diag_max_l == adt::kDiagAll) {
+          fbest = ms;
+          open.insert(it->first);
+        }
+      }
     }
     if (flags & ADT_ADJOINT) {
       abest = 3.4e38f;
@@ -1529,7 +1758,7 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
   std::vector<adt_event3d> all(ev, ev + nev);
   const int wgs[3] = {256, 512, 1024};
   for (int order = 0; order < 2 && rc == ADT_OK; ++order) {
-    TuneSnap sn{cur.global, classes};
+    TuneSnap sn{cur.global, classes, open};
     sn.global.order = order;
     sn.global.fuse_max_n = 0;
     float fbest = 0.f, abest = 0.f;
@@ -1589,6 +1818,7 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune[tune_index<T>()] = win;
     g_classes[tune_index<T>()] = classes;
+    g_open[tune_index<T>()] = open;
   }
   if (best) *best = win;
   return ADT_OK;
@@ -1618,6 +1848,7 @@ int graph_create_impl(const adt_event3d* ev, int nev, int flags, GraphBase** out
   if (rc) return rc;
   if (mis && (rc = plan.attach_misfit(ev, nev, mis))) return rc;
   if (tn.order) plan.order_largest_first();
+  plan.plan_teams(flags, tn);
   GraphBase* g = new GraphBase();
   g->nev = nev;
   g->off_info = plan.off_info;
@@ -1630,6 +1861,9 @@ int graph_create_impl(const adt_event3d* ev, int nev, int flags, GraphBase** out
   char* base = (char*)g->ws;
   e = hipMemcpy(base + plan.off_desc, plan.descs.data(), sizeof(adt::EventDesc) * nev,
                 hipMemcpyHostToDevice);
+  if (e == hipSuccess && plan.team.on())
+    e = hipMemcpy(base + plan.team.off_desc, plan.team.descs.data(),
+                  sizeof(adt::TeamDesc) * plan.team.descs.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess && plan.mis) {
     rc = plan.upload_misfit(base, nev, nullptr);
     if (rc == ADT_OK) e = hipDeviceSynchronize();
@@ -1644,8 +1878,7 @@ int graph_create_impl(const adt_event3d* ev, int nev, int flags, GraphBase** out
   e = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
   if (e == hipSuccess) {
-    rc = launch_batch<T>((const adt::EventDesc*)(base + plan.off_desc), nev, flags, plan.mix, tn,
-                         (adt_info*)(base + plan.off_info), cs, plan.misfit_run(base));
+    rc = launch_batch<T>(plan, base, nev, flags, tn, cs, plan.misfit_run(base));
     hipError_t e2 = hipStreamEndCapture(cs, &g->graph);
     if (rc == ADT_OK && e2 != hipSuccess) e = e2;
   }
@@ -1701,6 +1934,7 @@ int adt_tune_class_set(int32_t dtype, int64_t m, int64_t n, int64_t l, const adt
   if (rc) return rc;
   if (t && !tune_valid(*t)) return fail(ADT_EINVAL, "tune_class_set: setting out of range");
   std::lock_guard<std::mutex> lk(g_tune_mu);
+  g_open[dtype].erase(class_of(m, n, l));
   if (t)
     g_classes[dtype][class_of(m, n, l)] = *t;
   else
@@ -1729,6 +1963,7 @@ int adt_tune_class_clear(int32_t dtype) {
   if (dtype != 0 && dtype != 1) return fail(ADT_EINVAL, "tune_class_clear: dtype must be 0 or 1");
   std::lock_guard<std::mutex> lk(g_tune_mu);
   g_classes[dtype].clear();
+  g_open[dtype].clear();
   return ADT_OK;
 }
 int adt_tune_save(const char* path) {
@@ -1741,7 +1976,7 @@ int adt_tune_save(const char* path) {
     bool first = true;
     for (int d = 0; d < 2; ++d)
       for (const auto& kv : g_classes[d]) {
-        txt += std::string(first ? "\n  " : ",\n  ") + tune_json(d, kv.second, &kv.first);
+        txt += std::string(first ? "\n  " : ",\n  ") + tune_json(d, kv.second, &kv.first, g_open[d].count(kv.first) > 0);
         first = false;
       }
   }
@@ -1764,12 +1999,14 @@ int adt_tune_load(const char* path) {
   adt_tune glob[2];
   bool have[2] = {false, false};
   std::map<ClassKey, adt_tune> cls[2];
-  int rc = parse_tune_json(txt, glob, have, cls);
+  std::set<ClassKey> open[2];
+  int rc = parse_tune_json(txt, glob, have, cls, open);
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(g_tune_mu);
   for (int d = 0; d < 2; ++d) {
     if (have[d]) g_tune[d] = glob[d];
     g_classes[d] = cls[d];
+    g_open[d] = open[d];
   }
   return ADT_OK;
 }

@@ -41,6 +41,44 @@ struct EventDesc {
   const double* ry;
   const double* rz;
   int64_t nrec;
+  // An event that fwd3_team_kernel solves: its words (device); the diagonal
+  // kernel then takes it only if the abort word is set.  NULL otherwise.
+  const int* team_words;
+};
+
+// An event of fwd3_team_kernel: bands of at most H rows of the shorter
+// horizontal axis, ns slabs of kTW segments along k, R = bands * ns regions,
+// E chunks of the error pass; words: its counters, zeroed before the launch.
+struct TeamDesc {
+  int ev;  // index of its EventDesc
+  int bands, H, ns, R, E;
+  int* words;
+};
+constexpr int kTW = 4;             // waves per workgroup
+constexpr int kTeamXcds = 16;      // XCD ids are below this
+constexpr int kTeamGroups = 256;   // groups of workgroups per XCD
+constexpr int kTeamOver = 1 << 20;  // state of a finished event
+constexpr int kTeamSeqShift = 22;  // a count is (sweep << 22) + diagonals
+constexpr uint64_t kTeamPatience = 3000000000ull;  // 30 s of the 100 MHz clock
+// Word indices (16 words = 64 bytes apart: each is polled by itself).
+enum {
+  kTeamTicket = 0,   // items drawn
+  kTeamState = 16,   // iterations finished, or kTeamOver
+  kTeamAbort = 32,   // 1: values beyond the fast solve, 2: a wait ran out
+  kTeamSwept = 48,   // regions that have finished an iteration's last sweep
+  kTeamErred = 64,   // chunks of the error passes done
+  kTeamKey = 80,     // error keys of even / odd iterations (two 64-bit words)
+  kTeamCounts = 96   // per region: diagonals in memory
+};
+constexpr size_t team_words(int R) { return (size_t)kTeamCounts + 16 * (size_t)R; }
+// State of one launch, zeroed before it; `list` holds kTeamXcds * nteam ints.
+struct TeamShared {
+  unsigned long long group[kTeamXcds][kTeamGroups];
+  int arrived[kTeamXcds * 16];
+  int owned[kTeamXcds * 16];
+  int next;
+  int pad[15];
+  int list[1];
 };
 
 // One 2D event.
@@ -118,11 +156,15 @@ constexpr size_t kAdjRecBytes = 4 * sizeof(T);
 constexpr int kDiagAll = 1 << 30;
 template <typename T, bool MIX>
 __global__ void fwd3_diag_kernel(const EventDesc* evs, int max_iter);
+// Several workgroups per event, all on one XCD (kernels_team.hip).
+template <typename T, bool MIX>
+__global__ void fwd3_team_kernel(const EventDesc* evs, const TeamDesc* teams, TeamShared* sh,
+                                 int nteam, int per_group, int max_iter);
 // Forward then adjoint of each event in one workgroup (every event on the
 // diagonal forward).
 template <typename T, bool MIX>
 __global__ void fwd_adj3_diag_kernel(const EventDesc* evs, int max_iter);
-__global__ void info_clear_kernel(adt_info* info, int n);
+__global__ void info_clear_kernel(adt_info* info, int n, int* words, int64_t nwords);
 template <typename T>
 __global__ void strided_copy_kernel(const T* src, T* dst, int64_t N, int64_t d1, int64_t d2,
                                     int64_t s0, int64_t s1, int64_t s2, int to_rowmajor);

@@ -981,6 +981,8 @@ __device__ __forceinline__ void fwd3_diag_event(const EventDesc& ev, int max_ite
   __shared__ unsigned long long last_nan;
   const int m = ev.m, n = ev.n, l = ev.l;
   if (!ev.fwd_diag) return;  // handled by the k-streaming kernel
+  // solved by the team kernel unless that one gave it up
+  if (ev.team_words && ev.team_words[kTeamAbort] == 0) return;
   const int64_t N = (int64_t)m * n * l;
   const uint64_t bytes = (uint64_t)N * sizeof(T);
   if (threadIdx.x < 2) flags[threadIdx.x] = 0;

@@ -14,9 +14,14 @@
 
 namespace adt {
 
-// Clears the per-event diagnostics before a launch writes its fields (a
-// kernel, not a memset, so that it can sit in a captured graph).
-__global__ void info_clear_kernel(adt_info* __restrict__ info, int n) {
+// Clears the per-event diagnostics before a launch writes its fields, and
+// the launch's nwords counters (a kernel, not a memset, so that it can sit in
+// a captured graph).
+__global__ void info_clear_kernel(adt_info* __restrict__ info, int n, int* __restrict__ words,
+                                  int64_t nwords) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nwords;
+       i += (int64_t)gridDim.x * blockDim.x)
+    words[i] = 0;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
     info[i] = adt_info{};
 }

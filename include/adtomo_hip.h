@@ -242,8 +242,10 @@ typedef struct adt_tune {
                          node over the whole event (the only one that fuses
                          with the forward, see fuse_max_n) */
   int32_t fwd_segs;   /* diagonal forward: the k axis is cut into fwd_segs
-                         segments of up to 8 nodes, one per wave (1..8; 0 =
-                         8), and swept in chunks of 8 * fwd_segs nodes */
+                         segments (one wave each, 1..8), and swept in chunks of
+                         8 * fwd_segs nodes; 0 (default): the library chooses,
+                         8 segments or, where events are few or uneven, several
+                         workgroups per event */
 } adt_tune;
 int adt_get_tune(int32_t dtype, adt_tune *out);
 int adt_set_tune(int32_t dtype, const adt_tune *t);
