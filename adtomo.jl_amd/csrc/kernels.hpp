@@ -185,6 +185,20 @@ template <typename T>
 __global__ void adj3_finish_kernel(const T* lam, const T* f, T h, int64_t N, T* grad_f);
 template <typename T>
 __global__ void fwd2_event_kernel(const Event2Desc* evs, int max_iter);
+// 2D forward by bands of rows, one wave each (at most 1024 rows): travel times
+// in LDS (kFwd2Lds bytes with their border), or in memory (MEM).
+template <typename T, bool MEM>
+__global__ void fwd2_band_kernel(Event2Desc ev, int max_iter);
+constexpr int kFwd2Lds = 150 * 1024;
+// 2D adjoint with its working values in LDS: a byte per node (adj2_codes bytes
+// with a row before and after), and with LAM the multipliers, in kAdj2Lds;
+// queue: 2 N ints.
+template <typename T, bool LAM>
+__global__ void adj2_lds_kernel(Event2Desc ev);
+constexpr int kAdj2Lds = 112 * 1024, kAdj2Q = 4096;
+__host__ __device__ constexpr int64_t adj2_codes(int64_t W, int64_t N) {
+  return (N + 2 * (W + 4) + 15) & ~int64_t(15);
+}
 template <typename T>
 __global__ void adj3_kahn_kernel(const EventDesc* evs);
 // Tile-ordered 3D adjoint: NW waves per event, at most MAXT tiles of 8^3
