@@ -241,9 +241,19 @@ int parse_tune_json(const std::string& txt, adt_tune glob[2], bool have_glob[2],
   return ADT_OK;
 }
 
+// The library's choice of forward kernel for a set of events whose setting
+// leaves it open (diagonal forward, fwd_segs 0).
+int device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 256;
+  return n > 0 ? n : 256;
+}
+
 // ------------------------------------------------------------- adjoint ---
 // Two adjoint traversals (adt_tune.adj_algo): over 8x8x8 tiles (0; events
-// of at most kTileLargeMax tiles) or node by node over the event (1).
+// of at most kTileMax tiles) or node by node over the event (1).
 
 int64_t tiles_of(int64_t m, int64_t n, int64_t l) {
   const int64_t e = adt::kTileEdge;
@@ -253,7 +263,7 @@ int64_t tiles_of(int64_t m, int64_t n, int64_t l) {
 // The traversal an event set takes: the requested one, or the node-level
 // one when some event has more tiles than the tile kernels hold.
 int adj_algo_for(int requested, int64_t max_tiles) {
-  return (requested == 0 && max_tiles <= adt::kTileLargeMax) ? 0 : 1;
+  return (requested == 0 && max_tiles <= adt::kTileMax) ? 0 : 1;
 }
 
 // Adjoint workspace of one event (bytes): the EventDesc lam, code and queue
@@ -261,9 +271,9 @@ int adj_algo_for(int requested, int64_t max_tiles) {
 template <typename T>
 void adj_ws_bytes(int algo, int64_t N, int64_t tiles, size_t* lam, size_t* code, size_t* queue) {
   if (algo == 0) {
-    *lam = sizeof(T) * size_t(N);  // multipliers
-    *code = size_t(N);             // upwind codes
-    *queue = 16 * size_t(tiles);   // per tile: external-edge count, rank, inverse, key
+    *lam = sizeof(T) * adt::kTileNodes * size_t(tiles);  // multipliers
+    *code = adt::kTileNodes * size_t(tiles);             // upwind codes
+    *queue = sizeof(int) * adt::adj_words(tiles);
   } else {
     *lam = adt::kAdjRecBytes<T> * size_t(N);  // per-node records
     *code = 2 * size_t(N);                    // 16-bit node states
@@ -271,23 +281,33 @@ void adj_ws_bytes(int algo, int64_t N, int64_t tiles, size_t* lam, size_t* code,
   }
 }
 
+// Words that a launch of the tile traversal over nev events shares.
+size_t adj_shared_bytes(int nev) {
+  return sizeof(adt::TeamShared) + sizeof(int) * (size_t)adt::kTeamXcds * (size_t)nev;
+}
+
+// shared: adj_shared_bytes(nev) of device memory, used by algo 0.
 template <typename T>
 void launch_adj(int algo, int64_t max_tiles, int nev, const adt::EventDesc* d, int adj_wg,
-                hipStream_t s) {
+                void* shared, hipStream_t s) {
   if (algo != 0) {
     adt::adj3_kahn_kernel<T><<<nev, adj_wg, 0, s>>>(d);
     return;
   }
-  if (max_tiles <= adt::kTileSmallMax) {
-    adt::adj3_tile_kernel<T, adt::kTileWavesSmall, adt::kTileSmallMax>
-        <<<nev, adt::kTileWavesSmall * 64, 0, s>>>(d);
-  } else if (std::is_same<T, double>::value) {
-    adt::adj3_tile_kernel<T, adt::kTileWavesLarge64, adt::kTileLargeMax>
-        <<<nev, adt::kTileWavesLarge64 * 64, 0, s>>>(d);
-  } else {
-    adt::adj3_tile_kernel<T, adt::kTileWavesLarge32, adt::kTileLargeMax>
-        <<<nev, adt::kTileWavesLarge32 * 64, 0, s>>>(d);
-  }
+  const int64_t per_wg = (max_tiles + adt::kAdjWaves - 1) / adt::kAdjWaves;  // a wave per tile
+  const int chunks = (int)std::max<int64_t>(1, std::min<int64_t>(per_wg, 8192 / nev));
+  adt::adj3_codes_kernel<T><<<chunks * nev, 256, 0, s>>>(d, chunks, (int*)shared,
+                                                         (int64_t)(adj_shared_bytes(nev) / sizeof(int)));
+  adt::adj3_seeds_kernel<T><<<chunks * nev, 256, 0, s>>>(d, chunks);
+  // workgroups: what the compute units hold (2 of FP64, 4 of FP32 by their
+  // LDS), shared out over the events an XCD has at a time
+  const int cus = device_cus(), xcds = std::max(1, cus / 32);
+  const int slots = (sizeof(T) == 8 ? 2 : 4) * cus / xcds;
+  const int here = std::min((nev + xcds - 1) / xcds, slots);
+  const int per_group = (int)std::max<int64_t>(1, std::min<int64_t>(slots / here, per_wg));
+  // (those beyond the groups of the first events help with them)
+  const int grid = xcds * (int)std::min<int64_t>(slots, here * per_wg);
+  adt::adj3_tile_kernel<T><<<grid, adt::kAdjWaves * 64, 0, s>>>(d, (adt::TeamShared*)shared, nev, per_group);
 }
 
 int check_dims3(int64_t m, int64_t n, int64_t l) {
@@ -374,16 +394,6 @@ void set_event_setting(adt::EventDesc& d, const adt_tune& t) {
 }
 
 // ---- several workgroups per event (fwd3_team_kernel)
-
-// The library's choice of forward kernel for a set of events whose setting
-// leaves it open (diagonal forward, fwd_segs 0).
-int device_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 256;
-  return n > 0 ? n : 256;
-}
 
 struct TeamPlan {
   std::vector<adt::TeamDesc> descs;  // words: byte offsets until bind()
@@ -652,7 +662,8 @@ int bwd3_impl(const T* g, const T* u, const T* u0, const T* f, T h, int64_t m, i
   a = ((a + 255) / 256) * 256;
   c = ((c + 255) / 256) * 256;
   q = ((q + 255) / 256) * 256;
-  if ((rc = ws.alloc(a + c + q + 256 + sizeof(adt_info), s))) return rc;
+  const size_t os = a + c + q + 256 + ((sizeof(adt_info) + 255) / 256) * 256;
+  if ((rc = ws.alloc(os + adj_shared_bytes(1), s))) return rc;
   char* base = (char*)ws.p;
   adt::EventDesc d{};
   d.m = (int)m;
@@ -674,7 +685,7 @@ int bwd3_impl(const T* g, const T* u, const T* u0, const T* f, T h, int64_t m, i
   d.info = (adt_info*)(base + od + 256);
   ADT_HIP(hipMemcpyAsync(base + od, &d, sizeof(d), hipMemcpyHostToDevice, s));
   launch_clear(d.info, 1, nullptr, 0, s);
-  launch_adj<T>(algo, tiles, 1, (const adt::EventDesc*)(base + od), tn.adj_wg, s);
+  launch_adj<T>(algo, tiles, 1, (const adt::EventDesc*)(base + od), tn.adj_wg, base + os, s);
   ADT_HIP(hipGetLastError());
   adt_info hinf{};
   ADT_HIP(hipMemcpyAsync(&hinf, d.info, sizeof(adt_info), hipMemcpyDeviceToHost, s));
@@ -1209,6 +1220,7 @@ struct BatchPlan {
   std::vector<adt::EventDesc> descs;
   size_t ws_bytes = 0;
   size_t off_desc = 0, off_info = 0;
+  size_t off_adj = 0;  // words shared by the tile traversal's workgroups
   KernelMix mix;
   // attached receiver misfit (attach_misfit): table and coordinates in the
   // workspace
@@ -1337,6 +1349,7 @@ struct BatchPlan {
     }
     off_desc = take(sizeof(adt::EventDesc) * (nev ? nev : 1));
     off_info = take(sizeof(adt_info) * (nev ? nev : 1));
+    off_adj = mix.tile ? take(adj_shared_bytes(nev)) : 0;
     ws_bytes = off;
     for (int e = 0; e < nev; ++e) {
       const adt_event3d& x = ev[e];
@@ -1452,11 +1465,11 @@ int launch_batch(const BatchPlan<T>& plan, char* base, int nev, int flags, const
   }
   if (flags & ADT_ADJOINT) {
     if (km.tile) {
-      launch_adj<T>(0, km.tile_max, nev, ddesc, tn.adj_wg, s);
+      launch_adj<T>(0, km.tile_max, nev, ddesc, tn.adj_wg, base + plan.off_adj, s);
       ADT_HIP(hipGetLastError());
     }
     if (km.node) {
-      launch_adj<T>(1, 0, nev, ddesc, tn.adj_wg, s);
+      launch_adj<T>(1, 0, nev, ddesc, tn.adj_wg, nullptr, s);
       ADT_HIP(hipGetLastError());
     }
   }
@@ -1765,7 +1778,7 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
     if (flags & ADT_ADJOINT) {
       abest = 3.4e38f;
       for (int algo = 0; algo < 2; ++algo) {
-        if (algo == 0 && tiles_of(x0.m, x0.n, x0.l) > adt::kTileLargeMax) continue;
+        if (algo == 0 && tiles_of(x0.m, x0.n, x0.l) > adt::kTileMax) continue;
         TuneSnap t1 = sc;
         t1.global.adj_algo = algo;
         float ms = 0.f;

@@ -201,15 +201,29 @@ __host__ __device__ constexpr int64_t adj2_codes(int64_t W, int64_t N) {
 }
 template <typename T>
 __global__ void adj3_kahn_kernel(const EventDesc* evs);
-// Tile-ordered 3D adjoint: NW waves per event, at most MAXT tiles of 8^3
-// nodes.  Workspace per event: lam = multipliers [N] (T), code = upwind codes
-// [N] (bytes), queue = per-tile external-edge counts [tiles] (int32).
-template <typename T, int NW, int MAXT>
-__global__ void adj3_tile_kernel(const EventDesc* evs);
-constexpr int kTileEdge = 8;
-constexpr int kTileSmallMax = 8192;   // tiles of the 8-wave FP64 variant
-constexpr int kTileLargeMax = 65536;  // tiles of the large-event variants
-constexpr int kTileWavesSmall = 8, kTileWavesLarge64 = 6, kTileWavesLarge32 = 8;
+// Tile-ordered 3D adjoint (kernels_adjoint_tile.hip), for events of at most
+// kTileMax tiles of 8^3 nodes: codes, first queue, traversal; `chunks`
+// workgroups per event prepare, groups of per_group resolve.  Workspace per
+// event, tile by tile: lam = multipliers (T), code = upwind codes (bytes), 512
+// each per tile; queue = adj_words(): header, a count per tile, the queue.
+template <typename T>
+__global__ void adj3_codes_kernel(const EventDesc* evs, int chunks, int* sh, int64_t sh_words);
+template <typename T>
+__global__ void adj3_seeds_kernel(const EventDesc* evs, int chunks);
+template <typename T>
+__global__ void adj3_tile_kernel(const EventDesc* evs, TeamShared* sh, int nev, int per_group);
+constexpr int kTileEdge = 8, kTileNodes = 512;
+constexpr int kTileMax = 65536;
+constexpr int kAdjWaves = 4;  // per workgroup
+// Header words (64 bytes apart): places of the queue drawn and filled, nodes
+// left, 1 when the event is over (2: a wait ran out), passes over tiles.
+enum { kAdjHead = 0, kAdjTail = 16, kAdjLeft = 32, kAdjOver = 48, kAdjPasses = 64, kAdjHdr = 80 };
+// Places of the queue: every tile once, and one for each wave that may wait.
+constexpr int kAdjWaiters = 4096;
+__host__ __device__ constexpr int adj_ring(int ntiles) { return ntiles + kAdjWaiters; }
+constexpr size_t adj_words(int64_t ntiles) {
+  return (size_t)kAdjHdr + (size_t)ntiles + (size_t)adj_ring((int)ntiles);
+}
 template <typename T>
 __global__ void adj2_kahn_kernel(const Event2Desc* evs);
 template <typename T>

@@ -6,7 +6,6 @@
 // graph is acyclic, so Kahn's algorithm solves the system exactly once per
 // node, pulling each node's feeders in a fixed order.
 #include "adjoint3.hpp"
-#include "adjoint3_tile.hpp"
 #include "adjoint_device.hpp"
 #include "kernels.hpp"
 
@@ -31,13 +30,6 @@ __global__ void __launch_bounds__(1024) adj3_kahn_kernel(const EventDesc* __rest
   const EventDesc& ev = evs[blockIdx.x];
   if (ev.adj_algo != 1) return;
   adj3_kahn_event<T, 2, 2>(ev);
-}
-
-template <typename T, int NW, int MAXT>
-__global__ void __launch_bounds__(NW * 64) adj3_tile_kernel(const EventDesc* __restrict__ evs) {
-  const EventDesc& ev = evs[blockIdx.x];
-  if (ev.adj_algo != 0) return;
-  adj3_tile_event<T, NW, MAXT>(ev);
 }
 
 // ----------------------------------------------------------------- 2D ---
@@ -154,10 +146,6 @@ __global__ void __launch_bounds__(1024) adj2_kahn_kernel(const Event2Desc* __res
 
 template __global__ void adj3_kahn_kernel<double>(const EventDesc*);
 template __global__ void adj3_kahn_kernel<float>(const EventDesc*);
-template __global__ void adj3_tile_kernel<double, kTileWavesSmall, kTileSmallMax>(const EventDesc*);
-template __global__ void adj3_tile_kernel<double, kTileWavesLarge64, kTileLargeMax>(const EventDesc*);
-template __global__ void adj3_tile_kernel<float, kTileWavesSmall, kTileSmallMax>(const EventDesc*);
-template __global__ void adj3_tile_kernel<float, kTileWavesLarge32, kTileLargeMax>(const EventDesc*);
 template __global__ void adj2_kahn_kernel<double>(const Event2Desc*);
 template __global__ void adj2_kahn_kernel<float>(const Event2Desc*);
 

@@ -57,6 +57,7 @@
 #include "buffer_ops.hpp"
 #include "eikonal_device.hpp"
 #include "kernels.hpp"
+#include "team_device.hpp"
 
 namespace adt {
 
@@ -72,29 +73,12 @@ constexpr int kRing = 8;     // diagonals of the k exchange in LDS
 template <typename T>
 constexpr int kTL = 16 / (int)sizeof(T);  // nodes of k per lane
 
-using words_t = gptr<int>;
-
-__device__ __forceinline__ int ld_dev(gptr<const int> p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_dev(words_t p, int v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ int add_dev(words_t p, int v) {
-  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ int ld_wg(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 __device__ __forceinline__ void st_wg(int* p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-// Words shared only within an event's XCD: plain stores (they reach its L2)
-// and read-modify-writes at its L2.
-__device__ __forceinline__ void st_xcd(words_t p, int v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 // The event is finished or aborted: nobody waits for its items any more.
 __device__ __forceinline__ bool gone(gptr<const int> words) {
   return ld_dev(&words[kTeamState]) >= kTeamOver || ld_dev(&words[kTeamAbort]) != 0;
@@ -116,9 +100,6 @@ struct TPatience {
     return true;
   }
 };
-// Keeps the compiler from moving memory accesses across.
-__device__ __forceinline__ void code_fence() { asm volatile("" ::: "memory"); }
-
 __device__ __forceinline__ double ld_old(rsrc_t r, uint32_t off, double) {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kAuxDev));
 }
@@ -557,67 +538,20 @@ __global__ void __launch_bounds__(kTW * 64, 4)
   __shared__ uint64_t red[kTW];
   __shared__ TDraw draw;
   __shared__ int rank_s;
-  unsigned xcc;
-  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-  xcc &= kTeamXcds - 1;
+  const unsigned xcc = xcd_id();
   const int p = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (threadIdx.x == 0) rank_s = add_dev((words_t)&sh->arrived[xcc * 16], 1);
   __syncthreads();
   const int rank = uni(rank_s);
-  int grp = rank / per_group;
-  grp = grp < kTeamGroups ? grp : kTeamGroups - 1;
-  unsigned long long* slot = &sh->group[xcc][grp];
-  int gen = 0;        // thread 0: the group generation it works on
-  int help = -1;      // thread 0: position in the XCD's list once no event is left to take
+  TeamClaim claim(sh, xcc, rank, per_group);
   int team = -1;
   for (;;) {
     // ---- an event to work on
     if (threadIdx.x == 0) {
-      if (team < 0 && help < 0) {
-        for (;;) {
-          unsigned long long g = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          const int gg = (int)(g >> 32);
-          const unsigned lo = (unsigned)g;
-          if (lo == 1u) {
-            __builtin_amdgcn_s_sleep(2);
-            continue;
-          }
-          if (gg > gen) {
-            gen = gg;
-            if (lo == 0xffffffffu) {
-              help = 0;
-            } else {
-              team = (int)lo - 2;
-            }
-            break;
-          }
-          // the generation this workgroup has finished (or none yet): take the next event
-          unsigned long long want = g;
-          const unsigned long long claim = ((unsigned long long)gg << 32) | 1ull;
-          if (__hip_atomic_compare_exchange_strong(slot, &want, claim, __ATOMIC_RELAXED,
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-            const int e = add_dev((words_t)&sh->next, 1);
-            const unsigned nlo = e < nteam ? (unsigned)(e + 2) : 0xffffffffu;
-            if (e < nteam) {
-              const int at = add_dev((words_t)&sh->owned[xcc * 16], 1);
-              st_dev((words_t)&sh->list[xcc * nteam + at], e + 1);
-            }
-            __hip_atomic_store(slot, ((unsigned long long)(gg + 1) << 32) | nlo, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
-      }
-      if (team < 0 && help >= 0) {
-        // help with the XCD's other events, starting at a place of its own
-        const int n = ld_dev((words_t)&sh->owned[xcc * 16]);
-        while (help < n && team < 0) {
-          const int at = (help + rank) % n;
-          const int e = ld_dev((words_t)&sh->list[xcc * nteam + at]) - 1;
-          ++help;
-          if (e >= 0 && !gone((words_t)teams[e].words)) team = e;
-        }
-      }
+      if (team < 0)
+        team = claim_event(sh, nteam, claim, [](int) { return true; },
+                           [&](int e) { return gone((words_t)teams[e].words); });
       draw.team = team;
       if (team >= 0) {
         draw.ticket = add_dev((words_t)&teams[team].words[kTeamTicket], 1);
