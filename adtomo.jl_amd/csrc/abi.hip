@@ -1051,7 +1051,22 @@ struct MisfitRun {
   const adt::MisfitNodes* nodes;
   const double *rx, *ry, *rz;
   int nrec;
+  int64_t max_n;  // nodes of the largest box
 };
+
+// Workgroups per array that fill `count` arrays of at most N elements.
+int fill_parts(int count, int64_t N) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(4096 / count, N / 2048));
+}
+
+template <typename T>
+void launch_misfit(const MisfitRun& r, int nitem, hipStream_t s) {
+  const int parts = fill_parts(nitem, r.max_n);
+  adt::misfit_kernel<T><<<nitem * (parts + 1), 256, 0, s>>>(r.table, r.nodes, r.rx, r.ry, r.rz, r.nrec, parts);
+  // a thread per node: at most 8 of each receiver
+  const int np = std::max(1, std::min(64, (8 * r.nrec + 255) / 256));
+  adt::misfit_nodes_kernel<T><<<nitem * np, 256, 0, s>>>(r.table, r.nodes, r.rx, r.ry, r.rz, np);
+}
 
 // The receivers of a misfit grouped by interpolation node, for each box
 // among its items (host side of the deterministic misfit gradient, see
@@ -1293,10 +1308,10 @@ struct BatchPlan {
     return rnodes.upload(base, nev, s);
   }
   MisfitRun misfit_run(char* base) const {
-    if (!mis) return MisfitRun{nullptr, nullptr, nullptr, nullptr, nullptr, 0};
+    if (!mis) return MisfitRun{};
     const double* dc = (const double*)(base + off_coords);
     return MisfitRun{(const adt_misfit3d*)(base + off_mis), rnodes.table(base), dc,
-                     dc + mis->nrec, dc + 2 * mis->nrec, (int)mis->nrec};
+                     dc + mis->nrec, dc + 2 * mis->nrec, (int)mis->nrec, mix.max_n};
   }
 
   // Each event takes the setting of its box class (or the global one).
@@ -1460,7 +1475,7 @@ int launch_batch(const BatchPlan<T>& plan, char* base, int nev, int flags, const
     }
   }
   if (mr.table) {  // the events' receiver misfit: its gradient is the adjoint source
-    adt::misfit_kernel<T><<<nev, 256, 0, s>>>(mr.table, mr.nodes, mr.rx, mr.ry, mr.rz, mr.nrec);
+    launch_misfit<T>(mr, nev, s);
     ADT_HIP(hipGetLastError());
   }
   if (flags & ADT_ADJOINT) {
@@ -2260,12 +2275,14 @@ int source_u0_impl(const adt_source3d* src, int32_t nsrc, const T* vel0, int64_t
                                     " outside the 1-based grid");
   }
   hipStream_t st = (hipStream_t)stream;
-  DevBuf tab;
-  if ((rc = tab.alloc(sizeof(adt_source3d) * nsrc, st))) return rc;
-  ADT_HIP(hipMemcpyAsync(tab.p, src, sizeof(adt_source3d) * nsrc, hipMemcpyHostToDevice, st));
-  ADT_HIP(hipStreamSynchronize(st));  // the table is the caller's host memory
-  adt::source_u0_kernel<T><<<nsrc, 256, 0, st>>>((const adt_source3d*)tab.p, vel0, (int)m, (int)n,
-                                                 (int)l, h);
+  constexpr int kPer = sizeof(adt::SourceTable::s) / sizeof(adt::SourceDesc);
+  for (int at = 0; at < nsrc; at += kPer) {
+    const int k = std::min(kPer, nsrc - at);
+    adt::SourceTable tab{};
+    std::copy(src + at, src + at + k, tab.s);
+    const int parts = fill_parts(k, m * n * l);
+    adt::source_u0_kernel<T><<<k * parts, 256, 0, st>>>(tab, vel0, (int)m, (int)n, (int)l, h, parts);
+  }
   ADT_HIP(hipGetLastError());
   return ADT_OK;
 }
@@ -2304,8 +2321,11 @@ int misfit_impl(const adt_misfit3d* items, int32_t nitem, const double* rx, cons
     ADT_HIP(hipMemcpyAsync(dc + 2 * nrec, rz, sizeof(double) * nrec, hipMemcpyHostToDevice, st));
   }
   if ((rc = rn.upload(base, nitem, st))) return rc;
-  adt::misfit_kernel<T><<<nitem, 256, 0, st>>>((const adt_misfit3d*)(base + o_tab), rn.table(base),
-                                                dc, dc + nrec, dc + 2 * nrec, (int)nrec);
+  int64_t max_n = 0;
+  for (int i = 0; i < nitem; ++i)
+    max_n = std::max(max_n, (int64_t)items[i].m * items[i].n * items[i].l);
+  launch_misfit<T>(MisfitRun{(const adt_misfit3d*)(base + o_tab), rn.table(base), dc, dc + nrec,
+                             dc + 2 * nrec, (int)nrec, max_n}, nitem, st);
   ADT_HIP(hipGetLastError());
   // the staged coordinates are host copies: wait before they go out of scope
   ADT_HIP(hipStreamSynchronize(st));
@@ -2354,17 +2374,19 @@ int smooth_impl(const T* fvar, int64_t m, int64_t n, int64_t l, int32_t sh, int3
   T* sgn = (T*)ws.p;
   T* partial = sgn + N;
   const T wgt = T(1) / T((double)sh * sh * sv);
-  adt::smooth_pass1_kernel<T><<<nb, 256, 0, st>>>(fvar, (int)m, (int)n, (int)l, sh / 2, sv / 2, wgt,
-                                                  sgn, partial);
-  ADT_HIP(hipGetLastError());
-  if (grad_fvar) {
-    adt::smooth_pass2_kernel<T><<<nb, 256, 0, st>>>(sgn, (int)m, (int)n, (int)l, sh / 2, sv / 2,
-                                                    wgt, lambda, grad_fvar, partial, nb, value);
-  } else {
-    // value only: one thread sums the block partials
-    adt::smooth_pass2_kernel<T><<<1, 1, 0, st>>>(sgn, (int)m, (int)n, (int)l, sh / 2, sv / 2, wgt,
-                                                 lambda, nullptr, partial, nb, value);
-  }
+  // the 3x3x3 window has a kernel of its own
+  auto run = [&](auto r) {
+    constexpr int R = decltype(r)::value;
+    adt::smooth_pass1_kernel<T, R><<<nb, 256, 0, st>>>(fvar, (int)m, (int)n, (int)l, sh / 2, sv / 2,
+                                                       wgt, sgn, partial);
+    // (value only: one workgroup, for the block partials)
+    adt::smooth_pass2_kernel<T, R><<<grad_fvar ? nb : 1, 256, 0, st>>>(
+        sgn, (int)m, (int)n, (int)l, sh / 2, sv / 2, wgt, lambda, grad_fvar, partial, nb, value);
+  };
+  if (sh == 3 && sv == 3)
+    run(std::integral_constant<int, 1>());
+  else
+    run(std::integral_constant<int, 0>());
   ADT_HIP(hipGetLastError());
   return ADT_OK;
 }
@@ -2393,7 +2415,7 @@ int slowness_grad_impl(const T* fvar, int64_t N, T scale, const T* grad_fs, T* g
     ADT_HIP(hipGetLastError());
   }
   if (grad_scale) {
-    adt::sum_partials_kernel<T><<<1, 64, 0, st>>>((const T*)ws.p, N > 0 ? nb : 0, grad_scale);
+    adt::sum_partials_kernel<T><<<1, 256, 0, st>>>((const T*)ws.p, N > 0 ? nb : 0, grad_scale);
     ADT_HIP(hipGetLastError());
   }
   return ADT_OK;
@@ -2406,12 +2428,21 @@ int sum_arrays_impl(const T* const* arrays, int32_t narr, int64_t N, T* out, voi
     if (!arrays[k]) return fail(ADT_EINVAL, "sum_arrays: NULL array");
   if (N == 0) return ADT_OK;
   hipStream_t st = (hipStream_t)stream;
-  DevBuf tab;
-  int rc;
-  if ((rc = tab.alloc(sizeof(T*) * narr, st))) return rc;
-  ADT_HIP(hipMemcpyAsync(tab.p, arrays, sizeof(T*) * narr, hipMemcpyHostToDevice, st));
-  ADT_HIP(hipStreamSynchronize(st));  // the pointer table is the caller's host memory
-  adt::sum_arrays_kernel<T><<<grid_for(N), 256, 0, st>>>((const T* const*)tab.p, narr, N, out);
+  constexpr int kPer = sizeof(adt::ArrayTable::a) / sizeof(void*);
+  adt::ArrayTable tab{};
+  DevBuf more;
+  if (narr > kPer) {
+    int rc;
+    if ((rc = more.alloc(sizeof(T*) * narr, st))) return rc;
+    ADT_HIP(hipMemcpyAsync(more.p, arrays, sizeof(T*) * narr, hipMemcpyHostToDevice, st));
+    ADT_HIP(hipStreamSynchronize(st));  // the pointer table is the caller's host memory
+  } else {
+    std::copy(arrays, arrays + narr, tab.a);
+  }
+  if (more.p)
+    adt::sum_arrays_kernel<T, true><<<grid_for(N), 256, 0, st>>>(tab, (const void* const*)more.p, narr, N, out);
+  else
+    adt::sum_arrays_kernel<T, false><<<grid_for(N), 256, 0, st>>>(tab, nullptr, narr, N, out);
   ADT_HIP(hipGetLastError());
   return ADT_OK;
 }

@@ -114,19 +114,32 @@ struct MisfitNodes {
   void* gj;
 };
 
+// Tables passed as kernel arguments (kernel arguments are at most 4 KB).
+struct SourceTable {
+  SourceDesc s[64];
+};
+struct ArrayTable {
+  const void* a[256];
+};
+static_assert(sizeof(SourceTable) <= 3584 && sizeof(ArrayTable) <= 3584, "kernel arguments");
+
 template <typename T>
-__global__ void source_u0_kernel(const SourceDesc* src, const T* vel0, int m, int n, int l, T h);
+__global__ void source_u0_kernel(SourceTable tab, const T* vel0, int m, int n, int l, T h, int parts);
 template <typename T>
 __global__ void misfit_kernel(const MisfitDesc* d, const MisfitNodes* nodes, const double* rx,
-                              const double* ry, const double* rz, int nrec);
+                              const double* ry, const double* rz, int nrec, int parts);
+template <typename T>
+__global__ void misfit_nodes_kernel(const MisfitDesc* d, const MisfitNodes* nodes, const double* rx,
+                                    const double* ry, const double* rz, int parts);
 template <typename T>
 __global__ void model_kernel(const T* x, const T* vel0, int64_t N, T* fvar, T* f);
-template <typename T>
-__global__ void sum_arrays_kernel(const T* const* in, int nin, int64_t N, T* out);
-template <typename T>
+template <typename T, bool MORE>
+__global__ void sum_arrays_kernel(ArrayTable tab, const void* const* more, int nin, int64_t N,
+                                  T* out);
+template <typename T, int R>
 __global__ void smooth_pass1_kernel(const T* fvar, int m, int n, int l, int rh, int rv, T wgt,
                                     T* sgn, T* partial);
-template <typename T>
+template <typename T, int R>
 __global__ void smooth_pass2_kernel(const T* sgn, int m, int n, int l, int rh, int rv, T wgt,
                                     T lambda, T* grad, const T* partial, int npart, T* value);
 template <typename T>

@@ -80,11 +80,13 @@ __device__ __forceinline__ T trilinear_adjoint_at(const Trilinear<T>& t, T g, in
 // (the weights are >= 0) and leave the sum unchanged (a sum that starts at
 // +0 is never -0).
 //
-// Run by one workgroup of at least 256 threads: every thread zeroes grad_u,
-// the first 256 take the receivers (receiver j on thread j mod 256), so the
-// loss is summed in the same order whatever the workgroup size.
+// misfit_seeds: one workgroup of at least 256 threads; the first 256 take the
+// receivers (receiver j on thread j mod 256), so the loss is summed in the same
+// order whatever the workgroup size.  misfit_nodes: the node sums on threads
+// first, first + step, ... of any number of workgroups, once the seeds are in
+// memory.  misfit_event: all of it by one workgroup, grad_u zeroed first.
 template <typename T>
-__device__ __forceinline__ void misfit_event(const MisfitDesc& s, const MisfitNodes& nodes,
+__device__ __forceinline__ void misfit_seeds(const MisfitDesc& s, const MisfitNodes& nodes,
                                              const double* __restrict__ rx,
                                              const double* __restrict__ ry,
                                              const double* __restrict__ rz, int nrec) {
@@ -93,14 +95,9 @@ __device__ __forceinline__ void misfit_event(const MisfitDesc& s, const MisfitNo
   const T* __restrict__ u = (const T*)s.u;
   const T* __restrict__ tobs = (const T*)s.tobs;
   const T* __restrict__ w = (const T*)s.weight;
-  T* grad_u = (T*)s.grad_u;
   T* tcal = (T*)s.tcal;
   T* gj = (T*)nodes.gj;
   const T delta = (T)s.huber_delta;
-  const int64_t N = (int64_t)s.m * s.n * s.l;
-  if (grad_u)
-    for (int64_t p = threadIdx.x; p < N; p += blockDim.x) grad_u[p] = T(0);
-  __syncthreads();
   T acc = T(0);
   const int rt = threadIdx.x < kRecThreads ? (int)threadIdx.x : nrec;  // others take none
   for (int j = rt; j < nrec; j += kRecThreads) {
@@ -123,28 +120,50 @@ __device__ __forceinline__ void misfit_event(const MisfitDesc& s, const MisfitNo
       acc = acc + w[j] * rho;
       seed = -(w[j] * drho);
     }
-    if (grad_u) gj[j] = seed;
+    if (s.grad_u) gj[j] = seed;
   }
   if (threadIdx.x < kRecThreads) part[threadIdx.x] = acc;
-  __syncthreads();  // seeds (and the zeroed grad_u) before the node sums
-  if (grad_u) {
-    for (int64_t q = threadIdx.x; q < nodes.nuniq; q += blockDim.x) {
-      T sum = T(0);
-      for (int64_t e = nodes.off[q]; e < nodes.off[q + 1]; ++e) {
-        const int64_t en = nodes.ent[e];
-        const int64_t j = en >> 3;
-        const Trilinear<T> tr = trilinear_setup<T>(rx[j], ry[j], rz[j], s.n, s.l);
-        sum = sum + trilinear_adjoint_at(tr, gj[j], (int)(en >> 2) & 1, (int)(en >> 1) & 1,
-                                         (int)en & 1);
-      }
-      grad_u[nodes.node[q]] = sum;
-    }
-  }
+  __syncthreads();
   for (int off = kRecThreads / 2; off > 0; off >>= 1) {
     if ((int)threadIdx.x < off) part[threadIdx.x] = part[threadIdx.x] + part[threadIdx.x + off];
     __syncthreads();
   }
   if (threadIdx.x == 0) *(T*)s.loss = part[0];
+}
+
+template <typename T>
+__device__ __forceinline__ void misfit_nodes(const MisfitDesc& s, const MisfitNodes& nodes,
+                                             const double* __restrict__ rx,
+                                             const double* __restrict__ ry,
+                                             const double* __restrict__ rz, int first, int step) {
+  T* const grad_u = (T*)s.grad_u;
+  if (!grad_u) return;
+  const T* const gj = (const T*)nodes.gj;
+  for (int64_t q = first; q < nodes.nuniq; q += step) {
+    T sum = T(0);
+    for (int64_t e = nodes.off[q]; e < nodes.off[q + 1]; ++e) {
+      const int64_t en = nodes.ent[e];
+      const int64_t j = en >> 3;
+      const Trilinear<T> tr = trilinear_setup<T>(rx[j], ry[j], rz[j], s.n, s.l);
+      sum = sum + trilinear_adjoint_at(tr, gj[j], (int)(en >> 2) & 1, (int)(en >> 1) & 1,
+                                       (int)en & 1);
+    }
+    grad_u[nodes.node[q]] = sum;
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void misfit_event(const MisfitDesc& s, const MisfitNodes& nodes,
+                                             const double* __restrict__ rx,
+                                             const double* __restrict__ ry,
+                                             const double* __restrict__ rz, int nrec) {
+  T* const grad_u = (T*)s.grad_u;
+  const int64_t N = (int64_t)s.m * s.n * s.l;
+  if (grad_u)
+    for (int64_t p = threadIdx.x; p < N; p += blockDim.x) grad_u[p] = T(0);
+  misfit_seeds<T>(s, nodes, rx, ry, rz, nrec);
+  __syncthreads();  // seeds and the zeroed grad_u before the node sums
+  misfit_nodes<T>(s, nodes, rx, ry, rz, threadIdx.x, blockDim.x);
 }
 
 }  // namespace adt
