@@ -271,7 +271,7 @@ int adj_algo_for(int requested, int64_t max_tiles) {
 template <typename T>
 void adj_ws_bytes(int algo, int64_t N, int64_t tiles, size_t* lam, size_t* code, size_t* queue) {
   if (algo == 0) {
-    *lam = sizeof(T) * adt::kTileNodes * size_t(tiles);  // multipliers
+    *lam = sizeof(T) * (adt::kTileNodes + 2 * adt::kTileFaces) * size_t(tiles);  // multipliers, faces
     *code = adt::kTileNodes * size_t(tiles);             // upwind codes
     *queue = sizeof(int) * adt::adj_words(tiles);
   } else {
@@ -285,6 +285,13 @@ void adj_ws_bytes(int algo, int64_t N, int64_t tiles, size_t* lam, size_t* code,
 size_t adj_shared_bytes(int nev) {
   return sizeof(adt::TeamShared) + sizeof(int) * (size_t)adt::kTeamXcds * (size_t)nev;
 }
+
+// Up to this many workgroups per event its waves pick their tiles from a window
+// of the queue: with few waves the queue is long and every visit counts (256
+// events of 128x128x64, 2 workgroups each: 15.3 -> 12.7 ms), with many the waves
+// idle and would only get into each other's way (one event of 400x400x160, 64
+// workgroups: 22 -> 32 ms).
+constexpr int kPickGroup = 4;
 
 // shared: adj_shared_bytes(nev) of device memory, used by algo 0.
 template <typename T>
@@ -307,7 +314,8 @@ void launch_adj(int algo, int64_t max_tiles, int nev, const adt::EventDesc* d, i
   const int per_group = (int)std::max<int64_t>(1, std::min<int64_t>(slots / here, per_wg));
   // (those beyond the groups of the first events help with them)
   const int grid = xcds * (int)std::min<int64_t>(slots, here * per_wg);
-  adt::adj3_tile_kernel<T><<<grid, adt::kAdjWaves * 64, 0, s>>>(d, (adt::TeamShared*)shared, nev, per_group);
+  adt::adj3_tile_kernel<T><<<grid, adt::kAdjWaves * 64, 0, s>>>(d, (adt::TeamShared*)shared, nev, per_group,
+                                                                per_group <= kPickGroup);
 }
 
 int check_dims3(int64_t m, int64_t n, int64_t l) {

@@ -218,22 +218,25 @@ __global__ void adj3_kahn_kernel(const EventDesc* evs);
 // kTileMax tiles of 8^3 nodes: codes, first queue, traversal; `chunks`
 // workgroups per event prepare, groups of per_group resolve.  Workspace per
 // event, tile by tile: lam = multipliers (T), code = upwind codes (bytes), 512
-// each per tile; queue = adj_words(): header, a count per tile, the queue.
+// each per tile, and behind the multipliers travel times and multipliers of the k
+// faces, 128 each; queue = adj_words(): header, a count per tile, the queue.
 template <typename T>
 __global__ void adj3_codes_kernel(const EventDesc* evs, int chunks, int* sh, int64_t sh_words);
 template <typename T>
 __global__ void adj3_seeds_kernel(const EventDesc* evs, int chunks);
 template <typename T>
-__global__ void adj3_tile_kernel(const EventDesc* evs, TeamShared* sh, int nev, int per_group);
-constexpr int kTileEdge = 8, kTileNodes = 512;
+__global__ void adj3_tile_kernel(const EventDesc* evs, TeamShared* sh, int nev, int per_group,
+                                 bool pick);
+constexpr int kTileEdge = 8, kTileNodes = 512, kTileFaces = 128;
 constexpr int kTileMax = 65536;
 constexpr int kAdjWaves = 4;  // per workgroup
 // Header words (64 bytes apart): places of the queue drawn and filled, nodes
 // left, 1 when the event is over (2: a wait ran out), passes over tiles.
 enum { kAdjHead = 0, kAdjTail = 16, kAdjLeft = 32, kAdjOver = 48, kAdjPasses = 64, kAdjHdr = 80 };
-// Places of the queue: every tile once, and one for each wave that may wait.
+// Places of the queue: every tile once and one for each wave that may wait; with
+// more, a place is seldom used twice (which costs the check that it is empty).
 constexpr int kAdjWaiters = 4096;
-__host__ __device__ constexpr int adj_ring(int ntiles) { return ntiles + kAdjWaiters; }
+__host__ __device__ constexpr int adj_ring(int ntiles) { return 8 * ntiles + kAdjWaiters; }
 constexpr size_t adj_words(int64_t ntiles) {
   return (size_t)kAdjHdr + (size_t)ntiles + (size_t)adj_ring((int)ntiles);
 }

@@ -18,7 +18,9 @@
 // and tells the neighbouring tiles that it has resolved a feeder of theirs.  Codes
 // and multipliers are kept tile by tile (512 entries each, i j k order), so a
 // tile is one contiguous piece; a multiplier that is not final holds a NaN of
-// its own (kOpen), so the value is its own flag.
+// its own (Raw::open), so the value is its own flag.  The k faces of a tile, whose
+// nodes each lie in another 64-byte sector, are kept a second time, travel times
+// and multipliers, so that a neighbour reads 64 nodes in 8 sectors.
 //
 // Inside a tile lane (i, j) owns the row k = 0..7.  What is resolved, what
 // feeds what and along which sides are 8-bit masks in registers; the lanes
@@ -28,8 +30,8 @@
 //
 // Scheduling.  Each tile counts the deliveries it has not yet taken account
 // of; the delivery that finds the count at zero puts the tile in the event's
-// queue, so a tile is in the queue or with a wave, never twice.  (A tile with
-// feeders still to come may be put back while others wait, see kFew.)  A wave that
+// queue, so a tile is in the queue or with a wave, never twice.  (A tile
+// with feeders still to come may be put back while others wait, see kWindow.)  A wave that
 // takes it reads the count, then the halo, and afterwards takes the count it
 // read away: if anything was delivered meanwhile it goes on with the tile, the
 // halo's multipliers read anew.  The queue starts with the tiles that hold a
@@ -44,11 +46,11 @@
 //
 // What bounds it.  One event: the chain of tiles along the rays, for each a load
 // (5000 cycles), some 25 rounds of 900 cycles (LDS reads, six products in order,
-// a division) and the hand-over (4000).  Many events: the reads of the passes, of
-// which a k face costs a sector per node.  Measured, prepare and solve, against one
-// workgroup per event with its scheduling in LDS: 128x128x64 FP64 12.7 -> 1.8 ms,
-// 200x200x80 43 -> 5 ms, 400x400x160 460 -> 22 ms; 64 events of 128x128x64 FP32
-// 14.6 -> 4.5 ms; 256 of them FP64 17.1 -> 15.3 ms.
+// a division) and the hand-over (4000).  Many events: the latency of a pass's
+// dependent memory accesses with two waves a SIMD (LDS holds no more).  Measured,
+// prepare and solve, against one workgroup per event with its scheduling in LDS:
+// 128x128x64 FP64 12.7 -> 1.8 ms, 200x200x80 43 -> 4 ms, 400x400x160 460 -> 21 ms;
+// 64 events of 128x128x64 FP32 14.6 -> 4.5 ms; 256 of them FP64 17.1 -> 12.7 ms.
 #include "adjoint3.hpp"
 #include "buffer_ops.hpp"
 #include "eikonal_device.hpp"
@@ -61,19 +63,22 @@ namespace {
 
 constexpr int kT = 8;                   // tile edge (nodes)
 constexpr int kTN = kT * kT * kT;       // nodes per tile
+constexpr int kFaces = 2 * kT * kT;     // nodes of its k faces
+static_assert(kTileNodes == kTN && kTileFaces == kFaces, "tile workspace");
 constexpr int kBJ = kT + 2, kBI = kBJ * kBJ, kBox = kBI * kBJ;  // box with halo: strides, size
 constexpr uint64_t kAllZ = 0x4040404040404040ull;  // a row of Z codes (or of no nodes)
 // Word of a tile: deliveries not yet taken account of (16 bits); edges into it
 // from unresolved nodes of other tiles (10 bits); it has been worked on before.
 constexpr int kCountMask = 0xffff, kEdge = 1 << 16, kEdgeMask = 0x3ff, kSeen = 1 << 30;
-// Queue entry: tile + 1 (24 bits), times it was put back, kSeen.
-constexpr int kTileMask = 0xffffff, kBack = 1 << 24, kBackMask = 0x3f;
-// A tile of more than kFew edges that are still to come goes back to the end of
-// the queue, up to kBacks times, while the queue holds kLong others.  On 256
-// events of 128x128x64 (8 waves each) that makes 2.2 passes a tile instead of
-// 3.9: 12.6 ms instead of 16.5.  16 and 96 edges: 13.5 and 15.5 ms; a single event
-// has idle waves and no queue, where the early visits are free.
-constexpr int kFew = 48, kBacks = 4, kLong = 2;
+// Queue entry: tile + 1 (24 bits), kSeen.
+constexpr int kTileMask = 0xffffff;
+// While the queue holds kLong tiles (`pick`) a wave takes kWindow of them at once, works on
+// the one with the fewest edges still to come and puts the others back; a tile
+// that it made ready itself it keeps only with at most kFew.  On 256 events of
+// 128x128x64 that makes 2.1 passes a tile instead of 4, on 200 of 200x200x80 2.3
+// instead of 4.6 (windows of 4, 8, 32, 64: 18.3, 16.8, 16.6, 17.4 ms whole calls
+// for the first against 16.6).
+constexpr int kWindow = 16, kLong = 20, kFew = 48;
 __device__ __forceinline__ int edges_of(int w) { return (w >> 16) & kEdgeMask; }
 constexpr int kWaves = kAdjWaves;
 
@@ -103,7 +108,7 @@ struct Ev {
   int nti, ntj, ntk, ntiles;
   T h;
   gptr<const T> u, u0, g, f;
-  gptr<T> gu0, gf, lam;
+  gptr<T> gu0, gf, lam, uface, lface;  // faces: per tile k = 0, k = 7, 64 nodes each
   gptr<uint8_t> code;
   words_t hdr, word, ring;
   int cap;
@@ -123,6 +128,8 @@ struct Ev {
     gu0 = (gptr<T>)ev.grad_u0;
     gf = (gptr<T>)ev.grad_f;
     lam = (gptr<T>)ev.lam;
+    uface = lam + (int64_t)ntiles * kTN;
+    lface = uface + (int64_t)ntiles * kFaces;
     code = (gptr<uint8_t>)ev.code;
     hdr = (words_t)ev.queue;
     word = hdr + kAdjHdr;
@@ -233,9 +240,9 @@ __device__ __forceinline__ Row row_masks(const Ev<T>& E, const Tile& X) {
 
 // Multiplier words as the event's XCD has them now.
 template <typename T>
-__device__ __forceinline__ typename Raw<T>::U ld_lam(const Ev<T>& E, int64_t at) {
+__device__ __forceinline__ typename Raw<T>::U ld_lam(gptr<const T> p) {
   using U = typename Raw<T>::U;
-  return __hip_atomic_load((gptr<const U>)E.lam + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __hip_atomic_load((gptr<const U>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Bounded wait (30 s): call with every unsuccessful poll; true when the time
@@ -252,27 +259,52 @@ struct Patience {
   }
 };
 
-// Puts an entry into the next place of the queue.
+__device__ __forceinline__ void give_up(const EventDesc& ev, words_t hdr) {
+  ev.info->fault = 1;
+  st_dev(&hdr[kAdjOver], 2);
+}
+
+// Puts an entry into place `at` of the queue, drawn before.
 template <typename T>
-__device__ __forceinline__ void put_entry(const Ev<T>& E, const EventDesc& ev, int entry) {
-  const int at = add_xcd(&E.hdr[kAdjTail], 1);
+__device__ __forceinline__ void put_entry(const Ev<T>& E, const EventDesc& ev, int at, int entry) {
   const words_t slot = &E.ring[(unsigned)at % (unsigned)E.cap];
-  Patience wait;  // the wave that drew this place one round ago empties it
-  while (ld_dev(slot) != 0) {
-    if (wait.over()) {
-      ev.info->fault = 1;
-      st_dev(&E.hdr[kAdjOver], 2);
-      break;
+  if ((unsigned)at >= (unsigned)E.cap) {
+    Patience wait;  // the wave that drew this place one round ago empties it
+    while (ld_dev(slot) != 0) {
+      if (wait.over()) {
+        give_up(ev, E.hdr);
+        break;
+      }
     }
   }
   st_xcd(slot, entry);
 }
 
+// The entry of this lane's place, once it is there (0: the event is over), out
+// of the queue.
+template <typename T>
+__device__ __forceinline__ int get_entry(const Ev<T>& E, const EventDesc& ev, int at) {
+  const words_t slot = &E.ring[(unsigned)at % (unsigned)E.cap];
+  Patience wait;
+  int entry;
+  for (;;) {
+    entry = ld_dev(slot);
+    const int over = ld_dev(&E.hdr[kAdjOver]);
+    if (over) return 0;
+    if (entry) break;
+    if (wait.over()) give_up(ev, E.hdr);
+  }
+  st_xcd(slot, 0);
+  return entry;
+}
+
 // The wave's work on the tile of `entry`, with `taken` deliveries to it, until
 // nothing more is delivered.  Returns the queue entry of a tile that it has
-// made ready and takes next, or 0.
+// made ready and takes next, with that tile's word, or 0.  `busy`: the queue is
+// long.
 template <typename T>
-__device__ int work_tile(const Ev<T>& E, const EventDesc& ev, Node<T>* const box, int entry, int taken) {
+__device__ int work_tile(const Ev<T>& E, const EventDesc& ev, Node<T>* const box, int entry, int taken,
+                         bool busy, int& keep_word) {
   using U = typename Raw<T>::U;
   const int lane = lane_id(), la = lane >> 3, lb = lane & 7;
   const Tile X = tile_of(E, (entry & kTileMask) - 1);
@@ -282,10 +314,12 @@ __device__ int work_tile(const Ev<T>& E, const EventDesc& ev, Node<T>* const box
                       tile_nb(E, X, 3), tile_nb(E, X, 4), tile_nb(E, X, 5)};
   U hw[6];
   auto load_halo = [&]() {
-    const int hx[6] = {7 * 64 + lane, lane, la * 64 + 56 + lb, la * 64 + lb, lane * 8 + 7, lane * 8};
+    const int hx[4] = {7 * 64 + lane, lane, la * 64 + 56 + lb, la * 64 + lb};
 #pragma unroll
-    for (int q = 0; q < 6; ++q)
-      hw[q] = ld_lam(E, nbt[q] >= 0 ? (int64_t)nbt[q] * kTN + hx[q] : base);
+    for (int q = 0; q < 4; ++q)
+      hw[q] = ld_lam<T>(E.lam + (nbt[q] >= 0 ? (int64_t)nbt[q] * kTN + hx[q] : base));
+    hw[4] = ld_lam<T>(E.lface + (nbt[4] >= 0 ? (int64_t)nbt[4] * kFaces + 64 + lane : 0));
+    hw[5] = ld_lam<T>(E.lface + (nbt[5] >= 0 ? (int64_t)nbt[5] * kFaces + lane : 0));
   };
   // ---- travel times of the box; sources and slowness of the tile
   int bx[14];
@@ -310,7 +344,12 @@ __device__ int work_tile(const Ev<T>& E, const EventDesc& ev, Node<T>* const box
       const bool on = gi >= 0 && gi < E.m && gj >= 0 && gj < E.n && gk >= 0 && gk < E.l;
       const int64_t x = (int64_t)gi * sI + (int64_t)gj * E.l + gk;
       const uint32_t off = boff<T>(on, x);
-      uv[s] = bload(ru, off, T(0));
+      if (s < 12)
+        uv[s] = bload(ru, off, T(0));
+      else if (s == 12)
+        uv[s] = E.uface[nbt[4] >= 0 ? (int64_t)nbt[4] * kFaces + 64 + lane : 0];
+      else
+        uv[s] = E.uface[nbt[5] >= 0 ? (int64_t)nbt[5] * kFaces + lane : 0];
       if (s < 8) {
         in[s] = on;
         gx[s] = x;
@@ -330,7 +369,7 @@ __device__ int work_tile(const Ev<T>& E, const EventDesc& ev, Node<T>* const box
   if (seen) {  // nodes resolved before, by any wave
     U w[8];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) w[s] = ld_lam(E, base + s * 64 + lane);
+    for (int s = 0; s < 8; ++s) w[s] = ld_lam<T>(E.lam + base + s * 64 + lane);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const uint64_t b = __ballot(w[s] != Raw<T>::open);
@@ -422,6 +461,10 @@ __device__ int work_tile(const Ev<T>& E, const EventDesc& ev, Node<T>* const box
           E.gf[gx[s]] = -lr * rhs;
         }
       }
+      // the k faces: this lane's row ends
+      const T l0 = box[row].l, l7 = box[row + 7].l;
+      if (now & 1u) E.lface[(int64_t)X.t * kFaces + lane] = l0 == l0 ? l0 : T(__builtin_nan(""));
+      if (now & 0x80u) E.lface[(int64_t)X.t * kFaces + 64 + lane] = l7 == l7 ? l7 : T(__builtin_nan(""));
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     const bool left = __ballot((R.nz & ~done) != 0) != 0;
@@ -488,9 +531,12 @@ __device__ int work_tile(const Ev<T>& E, const EventDesc& ev, Node<T>* const box
     if (m) {
       const int ent = (nt + 1) | (old & kSeen);
       const uint64_t m0 = __ballot(idle && edges_of(old) - rel <= kFew);
-      const int sel = again ? -1 : __builtin_ctzll(m0 ? m0 : m);
-      if (sel >= 0) keep = __builtin_amdgcn_readlane(ent, sel);
-      if (idle && lane != sel) put_entry(E, ev, ent);
+      const int sel = again ? -1 : m0 ? __builtin_ctzll(m0) : busy ? -1 : __builtin_ctzll(m);
+      if (sel >= 0) {
+        keep = __builtin_amdgcn_readlane(ent, sel);
+        keep_word = __builtin_amdgcn_readlane(old + add, sel);
+      }
+      if (idle && lane != sel) put_entry(E, ev, add_xcd(&E.hdr[kAdjTail], 1), ent);
     }
     if (!again) return keep;
   }
@@ -541,7 +587,14 @@ __global__ void __launch_bounds__(256)
         nj[s - 1][3] = E.u[x + kp];
       }
     }
-    const int64_t base = (int64_t)t * kTN + lane;
+    const int64_t base = (int64_t)t * kTN + lane, fb = (int64_t)t * kFaces + (lb ? 64 : 0) + la;
+    if (lb == 0 || lb == 7) {
+#pragma unroll
+      for (int s = 0; s < kT; ++s) {
+        E.uface[fb + s * 8] = own[s + 1];
+        *((gptr<typename Raw<T>::U>)E.lface + fb + s * 8) = Raw<T>::open;
+      }
+    }
 #pragma unroll
     for (int s = 0; s < kT; ++s) {
       const int i = i0 + s;
@@ -594,7 +647,8 @@ __global__ void __launch_bounds__(256)
 
 template <typename T>
 __global__ void __launch_bounds__(kWaves * 64, sizeof(T) == 8 ? 2 : 4)
-    adj3_tile_kernel(const EventDesc* __restrict__ evs, TeamShared* sh, int nev, int per_group) {
+    adj3_tile_kernel(const EventDesc* __restrict__ evs, TeamShared* sh, int nev, int per_group,
+                     bool pick) {
   __shared__ Node<T> box[kWaves][kBox];
   __shared__ int event_s, rank_s;
   const unsigned xcd = xcd_id();
@@ -617,38 +671,59 @@ __global__ void __launch_bounds__(kWaves * 64, sizeof(T) == 8 ? 2 : 4)
       ev.info->adj_converged = 1;
       st_dev(&E.hdr[kAdjOver], 1);
     }
-    int entry = 0;
+    int entry = 0, word = 0;
+    bool busy = false;
     for (;;) {
       if (!entry) {
-        int at = 0;
-        if (lane_id() == 0) at = add_xcd(&E.hdr[kAdjHead], 1);
-        const words_t slot = &E.ring[(unsigned)uni(at) % (unsigned)E.cap];
-        Patience wait;
-        bool over = false;
-        for (;;) {
-          entry = uni(ld_dev(slot));
-          over = uni(ld_dev(&E.hdr[kAdjOver])) != 0;
-          if (entry || over) break;
-          if (wait.over()) {
-            ev.info->fault = 1;
-            st_dev(&E.hdr[kAdjOver], 2);
+        const int lane = lane_id();
+        int at = -1;
+        if (busy) {  // a window of places that are filled, or being filled
+          if (lane == 0) {
+            int h = ld_dev(&E.hdr[kAdjHead]);
+            const int tail = ld_dev(&E.hdr[kAdjTail]);
+            if (tail - h >= kLong &&
+                __hip_atomic_compare_exchange_strong(&E.hdr[kAdjHead], &h, h + kWindow, __ATOMIC_RELAXED,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+              at = h;
           }
+          at = uni(at);
         }
-        if (over) break;
-        if (lane_id() == 0) st_xcd(slot, 0);
-      }
-      // a tile that waits for much, while others wait in the queue: back
-      const int word = uni(ld_dev(&E.word[(entry & kTileMask) - 1]));
-      if (edges_of(word) > kFew && ((entry / kBack) & kBackMask) < kBacks) {
-        const int head = uni(ld_dev(&E.hdr[kAdjHead])), tail = uni(ld_dev(&E.hdr[kAdjTail]));
-        if (tail - head >= kLong) {
-          if (lane_id() == 0) put_entry(E, ev, entry + kBack);
-          entry = 0;
-          continue;
+        if (at >= 0) {
+          int mine = 0, mw = 0;
+          unsigned key = ~0u;
+          if (lane < kWindow) {
+            mine = get_entry(E, ev, at + lane);
+            if (mine) mw = ld_dev(&E.word[(mine & kTileMask) - 1]);
+            key = mine ? (unsigned)edges_of(mw) << 8 | lane : ~0u;
+          }
+#pragma unroll
+          for (int o = 1; o < kWindow; o <<= 1) {
+            const unsigned k = __shfl_xor(key, o);
+            key = k < key ? k : key;
+          }
+          key = uni(key);
+          if (key == ~0u) break;  // over
+          const int sel = key & 0xff;
+          const bool back = lane < kWindow && lane != sel && mine != 0;
+          const uint64_t bm = __ballot(back);
+          int to = 0;
+          if (lane == 0) to = add_xcd(&E.hdr[kAdjTail], __builtin_popcountll(bm));
+          to = uni(to);
+          if (back) put_entry(E, ev, to + __builtin_popcountll(bm & ((1ull << lane) - 1)), mine);
+          entry = __builtin_amdgcn_readlane(mine, sel);
+          word = __builtin_amdgcn_readlane(mw, sel);
+        } else {
+          int head = 0;
+          if (lane == 0) head = add_xcd(&E.hdr[kAdjHead], 1);
+          head = uni(head);
+          entry = uni(get_entry(E, ev, head));
+          if (!entry) break;
+          word = uni(ld_dev(&E.word[(entry & kTileMask) - 1]));
+          busy = pick && uni(ld_dev(&E.hdr[kAdjTail])) - head >= kLong;
         }
       }
       code_fence();
-      entry = work_tile(E, ev, box[w], entry, word & kCountMask);
+      entry = work_tile(E, ev, box[w], entry, word & kCountMask, busy, word);
     }
     __syncthreads();
   }
@@ -657,7 +732,7 @@ __global__ void __launch_bounds__(kWaves * 64, sizeof(T) == 8 ? 2 : 4)
 #define ADT_ADJ3_TILE(T)                                                             \
   template __global__ void adj3_codes_kernel<T>(const EventDesc*, int, int*, int64_t); \
   template __global__ void adj3_seeds_kernel<T>(const EventDesc*, int);              \
-  template __global__ void adj3_tile_kernel<T>(const EventDesc*, TeamShared*, int, int);
+  template __global__ void adj3_tile_kernel<T>(const EventDesc*, TeamShared*, int, int, bool);
 ADT_ADJ3_TILE(double)
 ADT_ADJ3_TILE(float)
 #undef ADT_ADJ3_TILE
