@@ -407,6 +407,7 @@ struct TeamPlan {
   std::vector<adt::TeamDesc> descs;  // words: byte offsets until bind()
   size_t off_desc = 0, off_zero = 0, zero_bytes = 0;
   int per_group = 1, grid = 0;
+  bool wide = false;  // eight nodes of k per lane instead of 16 bytes
   bool on() const { return !descs.empty(); }
 
   template <typename T>
@@ -416,8 +417,8 @@ struct TeamPlan {
            std::max(d.m, d.n) < (1 << adt::kTeamSeqShift) - 64;
   }
   template <typename T>
-  static adt::TeamDesc geometry(const adt::EventDesc& d) {
-    const int64_t LW = 16 / (int64_t)sizeof(T);
+  static adt::TeamDesc geometry(const adt::EventDesc& d, bool wide) {
+    const int64_t LW = wide ? 8 : 16 / (int64_t)sizeof(T);
     adt::TeamDesc t{};
     const int Ma = std::min(d.m, d.n);
     t.bands = (Ma + 63) / 64;
@@ -432,7 +433,8 @@ struct TeamPlan {
   // Lays out the words of the events `use` (indices into evs) from byte
   // offset `off` on; returns the end.
   template <typename T>
-  size_t build(std::vector<adt::EventDesc>& evs, const std::vector<int>& use, size_t off) {
+  size_t build(std::vector<adt::EventDesc>& evs, const std::vector<int>& use, bool wide_, size_t off) {
+    wide = wide_;
     auto take = [&](size_t b) {
       const size_t o = off;
       off += ((b + 255) / 256) * 256;
@@ -444,7 +446,7 @@ struct TeamPlan {
     off_zero = take(sizeof(adt::TeamShared) + sizeof(int) * (size_t)adt::kTeamXcds * nt);
     int64_t maxR = 1;
     for (int e : use) {
-      adt::TeamDesc t = geometry<T>(evs[e]);
+      adt::TeamDesc t = geometry<T>(evs[e], wide);
       t.ev = e;
       t.words = (int*)take(sizeof(int) * adt::team_words(t.R));
       evs[e].team_words = t.words;
@@ -452,10 +454,12 @@ struct TeamPlan {
       descs.push_back(t);
     }
     zero_bytes = off - off_zero;
-    // workgroups: up to 4 per compute unit (the kernel's occupancy); an event
+    // workgroups: up to 4 per compute unit, 2 of the wide form (the kernels'
+    // occupancy; 3 of the wide form with spills are slower: 60 against 49 ms on 256
+    // events of 128x128x64); an event
     // has work for about 2.5 sweeps' regions at a time
     const int cus = device_cus(), xcds = std::max(1, cus / 32);
-    const int slots = 4 * cus / xcds;
+    const int slots = (wide ? 2 : 4) * cus / xcds;
     const int here = (nt + xcds - 1) / xcds;  // events per XCD at a time
     per_group = (int)std::max<int64_t>(1, std::min<int64_t>(slots / std::min(here, slots),
                                                           (5 * maxR + 1) / 2 + 1));
@@ -473,17 +477,62 @@ struct TeamPlan {
     const adt::TeamDesc* td = (const adt::TeamDesc*)(base + off_desc);
     adt::TeamShared* sh = (adt::TeamShared*)(base + off_zero);
     const int nt = (int)descs.size();
+    auto run = [&](auto kernel) {
+      kernel<<<grid, adt::kTW * 64, 0, s>>>(d, td, sh, nt, per_group, kMaxIter3);
+    };
     if constexpr (std::is_same<T, float>::value) {
       if (mix) {
-        adt::fwd3_team_kernel<float, true>
-            <<<grid, adt::kTW * 64, 0, s>>>(d, td, sh, nt, per_group, kMaxIter3);
+        run(wide ? adt::fwd3_team_kernel<float, true, true> : adt::fwd3_team_kernel<float, true, false>);
         return;
       }
     }
-    adt::fwd3_team_kernel<T, false>
-        <<<grid, adt::kTW * 64, 0, s>>>(d, td, sh, nt, per_group, kMaxIter3);
+    run(wide ? adt::fwd3_team_kernel<T, false, true> : adt::fwd3_team_kernel<T, false, false>);
   }
 };
+
+// Which forward kernel suits these events?  Each one's time for one iteration,
+// from the steps it takes (microseconds a step as measured on an MI355X; the
+// iteration counts are the same):
+//   one workgroup per event: bands * N_b + H + 6 steps per sweep and k chunk,
+//     2.4 us + 0.27 us per node of a lane, half as much again where every CU has
+//     an event (they share the memory);
+//   several: an event alone takes 4 (M_a + N_b) + 30 slabs + 80 steps (its
+//     sweeps overlap), many are bound by the wave steps of all of them, on the
+//     CUs of the XCDs that have an event.  With 16 bytes of k per lane 1.1 us a
+//     step and 0.44 us per CU for each wave step (accesses to the L2, 16 bytes
+//     each); with eight nodes 2.6 us and 0.72 us (the local solves).
+// Forward of one workgroup, 16 bytes, eight nodes, in ms: one event of 128x128x64
+// FP64 28, 5.5, 10; 16 of 101x90x47 27, 5.0, 8.1; 64 of 128x128x64 with FP32
+// storage 28, 18, 13.6; 256 uneven ones 47, 49, 26; 200 of 200x200x80 241, 347,
+// 141; 256 of 128x128x64 FP64 48, 136, 49.
+enum class Forward { kOne, kTeam, kWide };
+template <typename T>
+Forward choose_forward(const std::vector<adt::EventDesc>& descs) {
+  const int cus = device_cus(), xcds = std::max(1, cus / 32), nev = (int)descs.size();
+  const double used = (double)cus * std::min(1.0, (double)nev / xcds);
+  double dmax = 0, dsum = 0, tmax[2] = {0, 0}, tsum[2] = {0, 0};
+  for (const adt::EventDesc& d : descs) {
+    const double Ma = std::min(d.m, d.n), Nb = std::max(d.m, d.n);
+    double one = 0;
+    for (int w = 0; w < 2; ++w) {
+      const adt::TeamDesc t = TeamPlan::geometry<T>(d, w == 1);
+      const double segs = std::ceil(d.l / (w ? 8.0 : 16.0 / sizeof(T)));
+      tmax[w] = std::max(tmax[w], (4 * (Ma + Nb) + 30 * t.ns + 80) * (w ? 2.6 : 1.1));
+      tsum[w] += 8 * t.bands * (Nb + t.H - 1) * segs * (w ? 0.72 : 0.44);
+      if (w) continue;
+      for (int c = 0; c < d.l; c += 8 * kSegsMax) {
+        const int lw = (std::min(d.l - c, 8 * kSegsMax) + kSegsMax - 1) / kSegsMax;
+        one += 8 * (t.bands * Nb + t.H + 6) * (2.4 + 0.27 * lw);
+      }
+    }
+    dmax = std::max(dmax, one);
+    dsum += one;
+  }
+  const double td = std::max(dmax * (1 + 0.5 * std::min(1.0, (double)nev / cus)), 1.5 * dsum / cus);
+  const double t0 = std::max(tmax[0], tsum[0] / used), t1 = std::max(tmax[1], tsum[1] / used);
+  if (std::min(t0, t1) >= 0.9 * td) return Forward::kOne;
+  return t0 <= t1 ? Forward::kTeam : Forward::kWide;
+}
 
 void launch_clear(adt_info* infos, int nev, void* words, size_t bytes, hipStream_t s) {
   const size_t nw = bytes / sizeof(int);
@@ -522,12 +571,12 @@ int fwd3_impl(const T* u0, const T* f, T h, int64_t m, int64_t n, int64_t l, T t
   d.f = df;
   d.u = du;
   set_event_setting(d, tn);
-  // one event leaves all other compute units idle: several workgroups for it
   TeamPlan team;
   const size_t off_info = ((bytes + 255) / 256) * 256;
   const size_t off_desc = off_info + ((sizeof(adt_info) + 255) / 256) * 256;
   size_t end = off_desc + 256;
-  if (snap.leaves_open(m, n, l) && TeamPlan::fits<T>(d)) end = team.build<T>(ds, {0}, end);
+  const Forward how = snap.leaves_open(m, n, l) && TeamPlan::fits<T>(d) ? choose_forward<T>(ds) : Forward::kOne;
+  if (how != Forward::kOne) end = team.build<T>(ds, {0}, how == Forward::kWide, end);
   DevBuf ws;
   if ((rc = ws.alloc(end, s))) return rc;
   char* base = (char*)ws.p;
@@ -1207,37 +1256,6 @@ bool fused(int flags, const KernelMix& km, const adt_tune& tn) {
          !km.tile && km.max_n <= tn.fuse_max_n;
 }
 
-// Do several workgroups per event pay for these events?  Both kernels' times
-// for one iteration, from the steps they take (microseconds a step as measured
-// on an MI355X; the iteration counts are the same):
-//   one workgroup per event: bands * N_b + H + 6 steps per sweep and k chunk,
-//     2.4 us + 0.27 us per node of a lane, events in parallel over the CUs;
-//   team: an event alone takes 4 (M_a + N_b) + 30 slabs + 80 steps (its sweeps
-//     overlap) of 1.1 us; many events are bound by their 16-byte accesses to
-//     the L2, 0.44 us per CU for each wave step.
-// 256 events of 128x128x64 FP64: 37 ms against 130 ms; 64 with FP32 storage: 28
-// against 18 ms; one: 28 against 5.5 ms.
-template <typename T>
-bool team_pays(const std::vector<adt::EventDesc>& descs) {
-  const double cus = device_cus();
-  double dmax = 0, dsum = 0, tmax = 0, tsum = 0;
-  for (const adt::EventDesc& d : descs) {
-    const adt::TeamDesc t = TeamPlan::geometry<T>(d);
-    const double Ma = std::min(d.m, d.n), Nb = std::max(d.m, d.n);
-    double one = 0;
-    for (int c = 0; c < d.l; c += 8 * kSegsMax) {
-      const int lw = (std::min(d.l - c, 8 * kSegsMax) + kSegsMax - 1) / kSegsMax;
-      one += 8 * (t.bands * Nb + t.H + 6) * (2.4 + 0.27 * lw);
-    }
-    const double segs = (d.l * (double)sizeof(T) + 15) / 16;
-    dmax = std::max(dmax, one);
-    dsum += one;
-    tmax = std::max(tmax, (4 * (Ma + Nb) + 30 * t.ns + 80) * 1.1);
-    tsum += 8 * t.bands * (Nb + t.H - 1) * segs * 0.44;
-  }
-  return std::max(tmax, tsum / cus) < 0.9 * std::max(dmax, dsum / cus);
-}
-
 template <typename T>
 struct BatchPlan {
   std::vector<adt::EventDesc> descs;
@@ -1417,8 +1435,9 @@ struct BatchPlan {
       if (!descs[e].pad || !TeamPlan::fits<T>(descs[e])) return;
       use.push_back((int)e);
     }
-    if (!team_pays<T>(descs)) return;
-    ws_bytes = team.build<T>(descs, use, ws_bytes);
+    const Forward how = choose_forward<T>(descs);
+    if (how == Forward::kOne) return;
+    ws_bytes = team.build<T>(descs, use, how == Forward::kWide, ws_bytes);
   }
   void bind(char* base) {
     team.bind(base, descs);
@@ -1743,7 +1762,7 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
       ds[e].fwd_diag = 1;
       team_ok = team_ok && TeamPlan::fits<T>(ds[e]);
     }
-    team_ok = team_ok && team_pays<T>(ds);
+    team_ok = team_ok && choose_forward<T>(ds) != Forward::kOne;
   }
   std::map<ClassKey, adt_tune> classes = cur.classes;
   std::set<ClassKey> open = cur.open;

@@ -170,7 +170,7 @@ constexpr int kDiagAll = 1 << 30;
 template <typename T, bool MIX>
 __global__ void fwd3_diag_kernel(const EventDesc* evs, int max_iter);
 // Several workgroups per event, all on one XCD (kernels_team.hip).
-template <typename T, bool MIX>
+template <typename T, bool MIX, bool WIDE>
 __global__ void fwd3_team_kernel(const EventDesc* evs, const TeamDesc* teams, TeamShared* sh,
                                  int nteam, int per_group, int max_iter);
 // Forward then adjoint of each event in one workgroup (every event on the

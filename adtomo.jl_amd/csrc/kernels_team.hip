@@ -44,16 +44,27 @@
 // What bounds it.  One event: the latency of a step, about 2000 cycles of one
 // wave per SIMD (two dependent local solves 870, the neighbours' minima 300, the
 // next loads 270, progress checks and hand-over 580); 2700 where u and f exceed
-// the XCD's 4 MB L2.  Two nodes per lane, because four would make a step 1.55
+// the XCD's 4 MB L2.  Two FP64 nodes per lane, because four would make a step 1.55
 // times as long for 6% fewer of them.  Many events: the L2's rate of 16-byte
 // accesses from 64 different columns (about 0.44 us per wave step and CU).
-// Measured, forward alone against one workgroup per event: 128x128x64 FP64, 3
-// iterations, 28.3 -> 5.5 ms; 64x64x32 9.5 -> 1.8 ms; 64 events of 128x128x64
-// with FP32 storage 28 -> 18 ms.
+//
+// Many events are taken by the wide form: eight nodes of k per lane (a slab is
+// then 32 nodes), whose memory accesses cover whole 64-byte columns and change
+// hands between lanes in LDS, one step ahead.  Its steps are 2.3 times as long, so
+// an event alone takes twice the time, but the accesses cost a fifth, and what
+// bounds it is the local solves (0.72 us per wave step and CU, two waves a SIMD:
+// its registers allow no third, and one with spills is slower).
+//
+// Measured, forward alone, one workgroup per event -> 16 bytes -> eight nodes, ms:
+// 128x128x64 FP64 28.3, 5.5, 10; 64x64x32 9.5, 1.8, 4.5; 16 events of 400x400x160
+// with FP32 storage 1476, 196, 106; 64 of 128x128x64 with FP32 storage 27.6, 17.9,
+// 13.6; 200 of 200x200x80 FP64 241, 347, 141; 256 of 128x128x64 FP64 48, 136, 49.
 //
 // Values the fast local solve does not cover (NaN, -0, infinities, values of
 // 2^240 and more, discriminants below 2^-767) set the event's abort word; the
 // diagonal kernel launched behind this one then solves the event from u0.
+#include <type_traits>
+
 #include "buffer_ops.hpp"
 #include "eikonal_device.hpp"
 #include "kernels.hpp"
@@ -489,6 +500,365 @@ __device__ __forceinline__ bool team_sweep(const TItem<T>& S, TWatch W, int w, w
   return ok;
 }
 
+// ---- the wide form: eight nodes of k per lane
+//
+// Memory is read and written in 16-byte pieces, the NP pieces of a column by
+// neighbouring lanes (64 / NP columns an instruction), and the pieces change hands
+// in LDS.  Staging of a wave: 64 columns of NP pieces, those of FP64 rotated by
+// their column's number so that neither side has bank conflicts, and behind them
+// the rows beyond the band.
+constexpr int kTWide = 8;  // nodes of k per lane
+template <typename T>
+constexpr int kNP = kTWide * (int)sizeof(T) / 16;  // pieces of a column
+template <typename T>
+constexpr int kStage = 66 * kNP<T>;                // pieces of a staging area
+template <typename T>
+__device__ __forceinline__ int stage_rot(int col) {
+  return kNP<T> == 4 ? (col >> 2) & 3 : 0;
+}
+
+// What a step of the wide form reads, one step ahead.
+template <typename T>
+struct TWideFlight {
+  // piece lane % NP of columns j 64 / NP + lane / NP
+  u32x4 old[kNP<T>], f[kNP<T>];
+  u32x4 up, dn;  // the first NP lanes: pieces of the rows beyond the band
+  T xd, xc;
+  int have;
+};
+
+// Nodes of one column out of the staging area (`at`: its first piece; rot: its
+// rotation), canonical order; entries from cnt on are not used.
+template <typename T, bool FULL, bool FC>
+__device__ __forceinline__ void from_stage(T (&x)[kTWide], lptr<u32x4> st, int at, int rot, int cnt) {
+  constexpr int LW = kTWide, PER = 16 / (int)sizeof(T), NP = kNP<T>;
+  if constexpr (FULL) {
+#pragma unroll
+    for (int c = 0; c < NP; ++c) {
+      const u32x4 v = st[at + ((c + rot) & (NP - 1))];
+      const unsigned w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int m = c * PER + i, e = FC ? LW - 1 - m : m;
+        if constexpr (sizeof(T) == 8)
+          x[e] = __longlong_as_double((long long)(((uint64_t)w[2 * i + 1] << 32) | w[2 * i]));
+        else
+          x[e] = __uint_as_float(w[i]);
+      }
+    }
+  } else {
+    const lptr<T> q = (lptr<T>)st;
+#pragma unroll
+    for (int e = 0; e < LW; ++e) {
+      const int m = e < cnt ? (FC ? cnt - 1 - e : e) : 0;
+      x[e] = q[(at + ((m / PER + rot) & (NP - 1))) * PER + m % PER];
+    }
+  }
+}
+template <typename T, bool FULL, bool FC>
+__device__ __forceinline__ void to_stage(const T (&x)[kTWide], lptr<u32x4> st, int at, int rot, int cnt) {
+  constexpr int LW = kTWide, PER = 16 / (int)sizeof(T), NP = kNP<T>;
+  if constexpr (FULL) {
+#pragma unroll
+    for (int c = 0; c < NP; ++c) {
+      unsigned w[4];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int m = c * PER + i, e = FC ? LW - 1 - m : m;
+        if constexpr (sizeof(T) == 8) {
+          const uint64_t b = (uint64_t)__double_as_longlong(x[e]);
+          w[2 * i] = (unsigned)b;
+          w[2 * i + 1] = (unsigned)(b >> 32);
+        } else {
+          w[i] = __float_as_uint(x[e]);
+        }
+      }
+      u32x4 v;
+      v.x = w[0];
+      v.y = w[1];
+      v.z = w[2];
+      v.w = w[3];
+      st[at + ((c + rot) & (NP - 1))] = v;
+    }
+  } else {
+    const lptr<T> q = (lptr<T>)st;
+#pragma unroll
+    for (int e = 0; e < LW; ++e) {
+      const int m = FC ? cnt - 1 - e : e;
+      if (e < cnt) q[(at + ((m / PER + rot) & (NP - 1))) * PER + m % PER] = x[e];
+    }
+  }
+}
+
+// As team_sweep, with loads one step ahead: what a step consumes was issued
+// after the stores of the step two before it.
+template <typename T, bool MIX, bool FULL, bool FC>
+__device__ __forceinline__ bool team_sweep_wide(const TItem<T>& S, TWatch W, int w, words_t count,
+                                                words_t words, lptr<T> ring, lptr<u32x4> st,
+                                                uint64_t* prog, int* stop) {
+  constexpr int LW = kTWide;
+  constexpr int SZ = (int)sizeof(T), PER = 16 / SZ, NP = kNP<T>, CP = 64 / NP;
+  const int p = threadIdx.x & 63;
+  const int cnt = FULL ? LW : S.cnt;
+  const T inf = (T)__builtin_inf();
+  const bool lastw = w == S.nw - 1;
+  const int klo = S.k0 - 1, khi = S.k0 + cnt;
+  const bool has_cm = FC ? khi < S.l : klo >= 0;
+  const bool has_cp = FC ? klo >= 0 : khi < S.l;
+  const int dcm = FC ? cnt * SZ : -SZ, dcp = FC ? -SZ : cnt * SZ;
+  const bool mem_cm = w == 0 && has_cm;
+  const bool row = p < S.Hr;
+  const bool loads = row || (p == S.Hr && S.dn);
+  const bool edge64 = S.Hr == 64 && S.dn;
+  const int dC = S.dA - S.dB;  // bytes from a column to the next of its diagonal
+  int off = S.off0 + p * dC, b = -p;                    // the lane's column
+  int qoff = S.off0 + (p / NP) * dC + (p % NP) * 16;     // the lane's piece, first of four
+  int qb = -(p / NP);
+  const bool piece = FULL || (p % NP) * PER < cnt;       // (pieces past the segment: not read)
+  // (the rotation of column CP j + p / NP does not depend on j)
+  const int qat = (p / NP) * NP + ((p % NP + stage_rot<T>(p / NP)) & (NP - 1));  // its place in the staging area
+  const int at = p * NP, rot = stage_rot<T>(p);             // the lane's column there
+  auto sel = [](bool ok, int o) -> uint32_t { return ok ? (uint32_t)o : kOOB; };
+  bool unsafe = false;
+  auto wild = [&](const T (&x)[LW]) {
+    bool r = false;
+#pragma unroll
+    for (int e = 0; e < LW; ++e)
+      if (FULL || e < cnt) r = (int)r | (int)Real<T>::wild_(x[e]) | (int)Real<T>::odd_(x[e]);
+    return r;
+  };
+  auto in = [&](int bb) { return (unsigned)bb < (unsigned)S.Nb; };
+  auto ld_old4 = [&](u32x4 (&x)[NP], int o, int bb) {  // old values of the columns at (o, bb)
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const int col = CP * j + (p / NP);
+      const bool ok = piece && (col < S.Hr || (col == S.Hr && S.dn)) && in(bb - CP * j);
+      x[j] = __builtin_amdgcn_raw_buffer_load_b128(S.src, sel(ok, o + CP * j * dC), 0, kAuxDev);
+    }
+  };
+  auto put4 = [&](const u32x4 (&x)[NP]) {
+#pragma unroll
+    for (int j = 0; j < NP; ++j) st[qat + 64 * j] = x[j];
+  };
+  // what step v reads (v = the diagonal of off, b, qoff, qb plus k columns)
+  auto issue = [&](TWideFlight<T>& F, int v, int k) {
+    const bool ends = p < NP && piece;
+    if (S.up)
+      F.up = __builtin_amdgcn_raw_buffer_load_b128(
+          S.u, sel(ends && in(v), S.off0 + v * S.dB - S.dA + p * 16), 0, kAuxDev);
+    if (edge64)
+      F.dn = __builtin_amdgcn_raw_buffer_load_b128(
+          S.src, sel(ends && in(v - 63), S.off0 + v * S.dB + 63 * dC + S.dA + p * 16), 0, kAuxDev);
+    if (mem_cm) F.xc = ld_old(S.u, sel(in(b + k) && row, off + k * S.dB + dcm), T(0));
+    if (w == 0) F.have = ld_dev(W.ptr);
+    code_fence();
+    ld_old4(F.old, qoff + (k + 1) * S.dB, qb + k + 1);
+    code_fence();
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const bool ok = piece && CP * j + (p / NP) < S.Hr && in(qb + k - CP * j);
+      F.f[j] = __builtin_amdgcn_raw_buffer_load_b128(S.f, sel(ok, qoff + k * S.dB + CP * j * dC), 0, 0);
+    }
+    code_fence();
+    F.xd = ld_old(S.src, sel(in(b + k) && row && has_cp, off + k * S.dB + dcp), T(0));
+  };
+  // the diagonal's values out of the staging area into memory
+  auto st4 = [&](int o, int bb, bool on) {
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const bool ok = on && piece && CP * j + (p / NP) < S.Hr && in(bb - CP * j);
+      const u32x4 x = st[qat + 64 * j];
+      const uint32_t a = sel(ok, o + CP * j * dC);
+      if constexpr (FULL) {
+        __builtin_amdgcn_raw_buffer_store_b128(x, S.u, a, 0, 0);
+      } else {
+        const unsigned y[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          const uint32_t ai = ok && (p % NP) * PER + i < cnt ? a + (uint32_t)(i * SZ) : kOOB;
+          if constexpr (sizeof(T) == 8)
+            bstore(S.u, ai, __longlong_as_double((long long)(((uint64_t)y[2 * i + 1] << 32) | y[2 * i])));
+          else
+            bstore(S.u, ai, __uint_as_float(y[i]));
+        }
+      }
+    }
+  };
+
+  bool ok = true;
+  if (w == 0) {
+    ok = watch_wait(W, -1, p, words);
+    if (!ok) st_wg(stop, 1);
+  } else {
+    int d;
+    while (get_prog(&prog[w - 1], d) < 0) {
+      if (uni(ld_wg(stop))) {
+        ok = false;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  if (!ok) return false;
+  code_fence();
+  TWideFlight<T> F;
+  F.xc = inf;
+  T NEWP[LW], OWN[LW], OLDN[LW];  // new(v-1), old(v) -> new(v), old(v+1)
+  ld_old4(F.old, qoff, qb);
+  put4(F.old);
+  code_fence();
+  from_stage<T, FULL, FC>(OWN, st, at, rot, cnt);
+  code_fence();
+  issue(F, 0, 0);
+  code_fence();
+  st4(qoff, qb, false);
+  code_fence();
+  if (p == 0) put_prog(&prog[w], 0, 0);
+  {
+    const bool i0 = loads && in(b);
+    if (S.first) unsafe = (int)unsafe | (int)wild(OWN);
+#pragma unroll
+    for (int e = 0; e < LW; ++e) {
+      NEWP[e] = inf;
+      OLDN[e] = i0 ? OWN[e] : inf;
+    }
+  }
+  int dn_seen = 0;
+  for (int v = 0; v < S.V; ++v) {
+    uint64_t pr = 0;
+    T xr = inf;
+    if (w > 0) {
+      pr = __hip_atomic_load(&prog[w - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      code_fence();
+      xr = ring[((w - 1) * kRing + (v & (kRing - 1))) * 64 + p];
+    }
+    const bool in1 = loads && in(b + 1);
+    const bool val = row && in(b);
+    T ma[LW], f[LW];
+    {
+      T x[LW];
+      code_fence();
+      put4(F.old);
+      code_fence();
+      from_stage<T, FULL, FC>(x, st, at, rot, cnt);
+      code_fence();
+      put4(F.f);
+      code_fence();
+      from_stage<T, FULL, FC>(f, st, at, rot, cnt);
+      if (S.first) {
+        unsafe = (int)unsafe | (int)wild(x);
+        bool r = false;
+#pragma unroll
+        for (int e = 0; e < LW; ++e)
+          if (FULL || e < cnt) r = (int)r | (int)Real<T>::wild_(f[e]);
+        unsafe = (int)unsafe | (int)r;
+      }
+#pragma unroll
+      for (int e = 0; e < LW; ++e) {
+        OWN[e] = OLDN[e];
+        OLDN[e] = in1 ? x[e] : inf;
+      }
+      T eu[LW], ed[LW];
+#pragma unroll
+      for (int e = 0; e < LW; ++e) eu[e] = ed[e] = inf;
+      if (S.up) {
+        if (p < NP) st[64 * NP + p] = F.up;
+        code_fence();
+        from_stage<T, FULL, FC>(eu, st, 64 * NP, 0, cnt);
+      }
+      if (edge64) {
+        if (p < NP) st[65 * NP + p] = F.dn;
+        code_fence();
+        from_stage<T, FULL, FC>(ed, st, 65 * NP, 0, cnt);
+      }
+      code_fence();
+#pragma unroll
+      for (int e = 0; e < LW; ++e)
+        ma[e] = Real<T>::min1_(dpp_shift<kDppUp>(eu[e], NEWP[e]), dpp_shift<kDppDn>(ed[e], OLDN[e]));
+    }
+    const T xd = has_cp ? own_copy(F.xd) : inf;
+    T xc = own_copy(F.xc);
+    // these loads were issued after step v-2's stores, which are complete then
+    asm volatile("" ::"v"(OLDN[0]), "v"(f[0]), "v"(xd) : "memory");
+    int done = v - 1 > 0 ? v - 1 : 0;
+    if (w > 0) {
+      if (__builtin_expect(uni((int)(pr >> 32)) < v + 1, 0)) {
+        int d;
+        while (get_prog(&prog[w - 1], d) < v + 1 && ok) {
+          if (uni(ld_wg(stop))) ok = false;
+        }
+        pr = (unsigned)d;
+        code_fence();
+        xr = ring[((w - 1) * kRing + (v & (kRing - 1))) * 64 + p];
+      }
+      const int up_done = uni((int)(unsigned)pr);
+      done = done < up_done ? done : up_done;
+      xc = xr;
+    } else {
+      W.have = F.have;
+      const bool low = p < 5 && W.have < W.need(v - 1);
+      if (__builtin_amdgcn_ballot_w64(low) != 0 && ok && !watch_wait(W, v - 1, p, words)) {
+        st_wg(stop, 1);
+        ok = false;
+      }
+    }
+    code_fence();
+    issue(F, v + 1, 1);
+    // ---- the lane's nodes
+    if (val) {
+#pragma unroll
+      for (int e = 0; e < LW; ++e) {
+        if (FULL || e < cnt) {
+          const T cm = e == 0 ? xc : OWN[e == 0 ? 0 : e - 1];
+          const T cp = (FULL ? e + 1 < LW : e + 1 < cnt) ? OWN[e + 1 < LW ? e + 1 : e] : xd;
+          const T mc = Real<T>::min1_(cm, cp);
+          const T mb = Real<T>::min1_(NEWP[e], OLDN[e]);
+          T cand;
+          if constexpr (MIX)
+            cand = (T)solution3d<double, true>(ma[e], mb, mc, f[e], S.hd, unsafe);
+          else
+            cand = solution3d<T, true>(ma[e], mb, mc, f[e], S.h, unsafe);
+          unsafe = (int)unsafe | (int)Real<T>::odd_(cand);
+          OWN[e] = Real<T>::min1_(cand, OWN[e]);
+        }
+      }
+    }
+    if (!lastw) {
+      T xo = OWN[LW - 1];
+      if constexpr (!FULL) {
+#pragma unroll
+        for (int e = 0; e < LW; ++e)
+          if (e == cnt - 1) xo = OWN[e];
+      }
+      while (dn_seen < v - kRing + 1 && ok) {
+        int d;
+        dn_seen = get_prog(&prog[w + 1], d);
+        if (dn_seen < v - kRing + 1 && uni(ld_wg(stop))) ok = false;
+      }
+      ring[(w * kRing + (v & (kRing - 1))) * 64 + p] = xo;
+      code_fence();
+    }
+    if (p == 0) {
+      put_prog(&prog[w], v + 1, done);
+      if (lastw) st_xcd(count, S.seqbase + done);
+    }
+    code_fence();
+    to_stage<T, FULL, FC>(OWN, st, at, rot, cnt);
+    code_fence();
+    st4(qoff, qb, true);
+    code_fence();
+#pragma unroll
+    for (int e = 0; e < LW; ++e) NEWP[e] = OWN[e];
+    off += S.dB;
+    ++b;
+    qoff += S.dB;
+    ++qb;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (__builtin_amdgcn_ballot_w64(unsafe) != 0 && p == 0) st_xcd(&words[kTeamAbort], 1);
+  return ok;
+}
+
 // max |u - snapshot| over nodes [lo, hi) and the next snapshot = u.
 template <typename T>
 __device__ __forceinline__ uint64_t err_chunk(const T* u, const T* snap, T* dst, int64_t lo,
@@ -527,12 +897,13 @@ struct TDraw {
 
 }  // namespace
 
-template <typename T, bool MIX>
-__global__ void __launch_bounds__(kTW * 64, 4)
+template <typename T, bool MIX, bool WIDE>
+__global__ void __launch_bounds__(kTW * 64, WIDE ? 2 : 4)
     fwd3_team_kernel(const EventDesc* __restrict__ evs, const TeamDesc* __restrict__ teams,
                      TeamShared* sh, int nteam, int per_group, int max_iter) {
-  constexpr int LW = kTL<T>;
+  constexpr int LW = WIDE ? kTWide : kTL<T>;
   __shared__ T ring_s[kTW * kRing * 64];
+  __shared__ u32x4 stage_s[WIDE ? kTW * kStage<T> : 1];
   __shared__ uint64_t prog[kTW];
   __shared__ int stop;
   __shared__ uint64_t red[kTW];
@@ -686,16 +1057,26 @@ __global__ void __launch_bounds__(kTW * 64, 4)
         }
         const words_t count = &words[kTeamCounts + 16 * (rb * td.ns + rs) + (seq & 3)];
         const lptr<T> ring = (lptr<T>)ring_s;
+        auto sweep = [&](auto full, auto down) {
+          constexpr bool FULL = decltype(full)::value, FC = decltype(down)::value;
+          if constexpr (WIDE)
+            team_sweep_wide<T, MIX, FULL, FC>(S, W, w, count, words, ring,
+                                              (lptr<u32x4>)stage_s + w * kStage<T>, prog, &stop);
+          else
+            team_sweep<T, MIX, FULL, FC>(S, W, w, count, words, ring, prog, &stop);
+        };
+        const std::true_type yes;
+        const std::false_type no;
         if (S.cnt == LW) {
           if (fk)
-            team_sweep<T, MIX, true, true>(S, W, w, count, words, ring, prog, &stop);
+            sweep(yes, yes);
           else
-            team_sweep<T, MIX, true, false>(S, W, w, count, words, ring, prog, &stop);
+            sweep(yes, no);
         } else {
           if (fk)
-            team_sweep<T, MIX, false, true>(S, W, w, count, words, ring, prog, &stop);
+            sweep(no, yes);
           else
-            team_sweep<T, MIX, false, false>(S, W, w, count, words, ring, prog, &stop);
+            sweep(no, no);
         }
       }
       __syncthreads();  // every wave's stores are complete
@@ -751,11 +1132,15 @@ __global__ void __launch_bounds__(kTW * 64, 4)
   }
 }
 
-template __global__ void fwd3_team_kernel<double, false>(const EventDesc*, const TeamDesc*,
-                                                         TeamShared*, int, int, int);
-template __global__ void fwd3_team_kernel<float, false>(const EventDesc*, const TeamDesc*,
-                                                        TeamShared*, int, int, int);
-template __global__ void fwd3_team_kernel<float, true>(const EventDesc*, const TeamDesc*,
-                                                       TeamShared*, int, int, int);
+#define ADT_TEAM(T, MIX, WIDE)                                                                  \
+  template __global__ void fwd3_team_kernel<T, MIX, WIDE>(const EventDesc*, const TeamDesc*,    \
+                                                          TeamShared*, int, int, int);
+ADT_TEAM(double, false, false)
+ADT_TEAM(float, false, false)
+ADT_TEAM(float, true, false)
+ADT_TEAM(double, false, true)
+ADT_TEAM(float, false, true)
+ADT_TEAM(float, true, true)
+#undef ADT_TEAM
 
 }  // namespace adt
