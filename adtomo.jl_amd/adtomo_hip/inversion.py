@@ -144,6 +144,9 @@ class TravelTimeInversion:
             self.fwd = EikonalGraph(self.u0s, fs, hs, tols, compute_f64=compute_f64)
             self.adj = EikonalGraph(self.u0s, fs, hs, tols, grad_us=self.grad_us, forward=False,
                                     us=self.fwd.us)
+        # the gradient's way to the host: a copy into pageable memory goes in small
+        # staged pieces (300 us a megabyte and a half into fresh pages)
+        self.gstage = torch.empty(self.N, dtype=self.dt, pin_memory=True)
         self.nevals = 0
         self.last_loss = {}
 
@@ -151,15 +154,19 @@ class TravelTimeInversion:
     def slot_bytes(N, elem):
         """Device bytes of one solve slot: u0, u, dL/du, dL/du0 and dL/df
         (N elements each) plus the batched workspace: the forward snapshot
-        and the tile adjoint's multipliers (N elements each), its upwind
-        codes (N bytes) and per-tile counts (N/512 int32)."""
-        return N * (7 * elem + 1) + 4 * (N // 512 + 64)
+        (N elements), the tile adjoint's multipliers and faces (1.5 N elements),
+        its upwind codes (N bytes), and per tile its word and places of the queue
+        (N/512 tiles, nine int32 each)."""
+        return N * (15 * elem // 2 + 1) + 36 * (N // 512) + (64 << 10)
 
     def fitting_chunk(self, ns, nphases, N, elem, budget=0.8):
         """All stations if their slots fit in ``budget`` of the free device
         memory, else the largest number of stations per launch that does."""
         free, _ = self.torch.cuda.mem_get_info()
-        per_station = nphases * self.slot_bytes(N, elem)
+        # the adjoint's workspace counts whole tiles of 8^3 nodes
+        tiles = int(np.prod([-(-s // 8) for s in self.shape]))
+        per_station = nphases * (self.slot_bytes(N, elem) +
+                                 (512 * tiles - N) * (3 * elem // 2 + 1))
         return max(1, min(ns, int(budget * free // per_station)))
 
     def _u0_scale(self, phase):
@@ -234,14 +241,15 @@ class TravelTimeInversion:
         self.nevals += 1
         if not grad:
             return loss
-        g = np.empty(self.nparams)
+        g = torch.empty(self.nparams, dtype=torch.float64)
         if self.joint:
             gv = O.slowness_grad(self.fvar, vpvs, self.grad_f["S"], grad_fvar=grad_fvar)
             g[-1] = float(gv.cpu().numpy()[0])
         gf = self.grad_f["P"] if "P" in self.phases else None
         gx = O.model_grad(self.x, self.fvar, grad_f=gf, grad_fvar=grad_fvar)
-        g[:self.N] = gx.cpu().numpy().reshape(-1)
-        return loss, g
+        self.gstage.copy_(gx.view(-1))  # (waits)
+        g[:self.N].copy_(self.gstage)
+        return loss, g.numpy()
 
     def travel_times(self, phase="P"):
         """Travel times of the last chunk's forward, one (m, n, l) tensor per slot."""
