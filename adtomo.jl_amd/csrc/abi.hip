@@ -306,10 +306,11 @@ void launch_adj(int algo, int64_t max_tiles, int nev, const adt::EventDesc* d, i
   adt::adj3_codes_kernel<T><<<chunks * nev, 256, 0, s>>>(d, chunks, (int*)shared,
                                                          (int64_t)(adj_shared_bytes(nev) / sizeof(int)));
   adt::adj3_seeds_kernel<T><<<chunks * nev, 256, 0, s>>>(d, chunks);
-  // workgroups: what the compute units hold (2 of FP64, 4 of FP32 by their
-  // LDS), shared out over the events an XCD has at a time
+  // workgroups: two per compute unit (what the LDS holds of FP64; four of FP32 are
+  // slower: 16 events of 400x400x160 48 ms against 42), shared out over the events
+  // an XCD has at a time
   const int cus = device_cus(), xcds = std::max(1, cus / 32);
-  const int slots = (sizeof(T) == 8 ? 2 : 4) * cus / xcds;
+  const int slots = 2 * cus / xcds;
   const int here = std::min((nev + xcds - 1) / xcds, slots);
   const int per_group = (int)std::max<int64_t>(1, std::min<int64_t>(slots / here, per_wg));
   // (those beyond the groups of the first events help with them)
@@ -503,7 +504,7 @@ struct TeamPlan {
 //     each); with eight nodes 2.6 us and 0.72 us (the local solves).
 // Forward of one workgroup, 16 bytes, eight nodes, in ms: one event of 128x128x64
 // FP64 28, 5.5, 10; 16 of 101x90x47 27, 5.0, 8.1; 64 of 128x128x64 with FP32
-// storage 28, 18, 13.6; 256 uneven ones 47, 49, 26; 200 of 200x200x80 241, 347,
+// storage 28, 18, 12.2; 256 uneven ones 47, 49, 26; 200 of 200x200x80 241, 347,
 // 141; 256 of 128x128x64 FP64 48, 136, 49.
 enum class Forward { kOne, kTeam, kWide };
 template <typename T>

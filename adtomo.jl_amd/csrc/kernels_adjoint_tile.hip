@@ -646,7 +646,7 @@ __global__ void __launch_bounds__(256)
 }
 
 template <typename T>
-__global__ void __launch_bounds__(kWaves * 64, sizeof(T) == 8 ? 2 : 4)
+__global__ void __launch_bounds__(kWaves * 64, 2)
     adj3_tile_kernel(const EventDesc* __restrict__ evs, TeamShared* sh, int nev, int per_group,
                      bool pick) {
   __shared__ Node<T> box[kWaves][kBox];
