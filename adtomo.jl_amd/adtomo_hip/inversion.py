@@ -144,9 +144,9 @@ class TravelTimeInversion:
             self.fwd = EikonalGraph(self.u0s, fs, hs, tols, compute_f64=compute_f64)
             self.adj = EikonalGraph(self.u0s, fs, hs, tols, grad_us=self.grad_us, forward=False,
                                     us=self.fwd.us)
-        # the gradient's way to the host: a copy into pageable memory goes in small
-        # staged pieces (300 us a megabyte and a half into fresh pages)
-        self.gstage = torch.empty(self.N, dtype=self.dt, pin_memory=True)
+        # the gradient's way to the host, in pieces: a copy into fresh pageable
+        # memory is staged by the runtime at a tenth of the rate
+        self.gstage = torch.empty(min(self.N, 1 << 20), dtype=self.dt, pin_memory=True)
         self.nevals = 0
         self.last_loss = {}
 
@@ -247,8 +247,11 @@ class TravelTimeInversion:
             g[-1] = float(gv.cpu().numpy()[0])
         gf = self.grad_f["P"] if "P" in self.phases else None
         gx = O.model_grad(self.x, self.fvar, grad_f=gf, grad_fvar=grad_fvar)
-        self.gstage.copy_(gx.view(-1))  # (waits)
-        g[:self.N].copy_(self.gstage)
+        gx, step = gx.view(-1), self.gstage.numel()
+        for at in range(0, self.N, step):
+            piece = self.gstage[:min(step, self.N - at)]
+            piece.copy_(gx[at:at + step])  # (waits)
+            g[at:at + piece.numel()].copy_(piece)
         return loss, g.numpy()
 
     def travel_times(self, phase="P"):
