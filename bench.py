@@ -42,14 +42,14 @@ sys.path[:0] = [ROOT, os.path.join(ROOT, "adtomo.jl_amd")]
 HBM_PEAK_GBS = 8000.0
 FWD_KERNEL = "fwd3_diag_kernel<double, false>"
 ADJ_KERNEL = "adj3_kahn_kernel<double>"
-ADJ_TILE_KERNEL = "adj3_tile_kernel<double, 8, 8192>"
+ADJ_TILE_KERNEL = "adj3_tile_kernel<double>"  # and the two that prepare it
 FUSED_KERNEL = "fwd_adj3_diag_kernel<double, false>"
 # HBM bytes (read + write) per launch of each kernel on this workload (256
 # events, default setting), measured with rocprofv3 FETCH_SIZE / WRITE_SIZE
-# scaled by a copy kernel of known size and checked against the TCC EA
-# request counters; kernels not profiled at the current code report null
-TRAFFIC_SOURCE = "profiles/pmc_traffic_fwd3_diag_adj3_tile_256x128x128x64.md"
-TRAFFIC_BYTES_256 = {FWD_KERNEL: 122.87e9 + 53.99e9, ADJ_TILE_KERNEL: 37.91e9 + 7.98e9}
+# scaled by a copy kernel of known size; kernels not profiled at the current
+# code report null
+TRAFFIC_SOURCE = "profiles/headline_256x128x128x64.md"
+TRAFFIC_BYTES_256 = {FWD_KERNEL: 127.47e9 + 54.32e9, ADJ_TILE_KERNEL: 39.45e9 + 11.29e9}
 
 
 def log(*a):
