@@ -69,6 +69,7 @@
 #include "eikonal_device.hpp"
 #include "kernels.hpp"
 #include "team_device.hpp"
+#include "team_gate.hpp"
 
 namespace adt {
 
@@ -893,13 +894,6 @@ __device__ __forceinline__ uint64_t err_chunk(const T* u, const T* snap, T* dst,
   return key;
 }
 
-// What the workgroup does next (drawn by thread 0).
-struct TDraw {
-  int team;    // index of the event's team descriptor, -1: leave
-  int ticket;
-  int quit;    // the event is finished or aborted
-};
-
 }  // namespace
 
 template <typename T, bool MIX, bool WIDE>
@@ -945,23 +939,22 @@ __global__ void __launch_bounds__(kTW * 64, WIDE ? 2 : 4)
     const int per_it = 8 * td.R + td.E;
     const int ticket = uni(draw.ticket);
     const int it = ticket / per_it, rem = ticket - it * per_it;
-    bool quit = uni(draw.quit) || it >= max_iter;
     const bool sweep = rem < 8 * td.R;
     const int sw = rem / td.R;
-    // ---- the iteration before is over (first sweep), the sweeps are done (error pass)
-    if (!quit && (sweep ? (sw == 0 && it > 0) : true)) {
-      if (threadIdx.x == 0) {
-        const words_t word = &words[sweep ? kTeamState : kTeamSwept];
-        const int need = sweep ? it : td.R * (it + 1);
-        TPatience wait;
-        while (ld_dev(word) < need)
-          if (wait.over(words)) break;
-        if (gone(words)) draw.quit = 1;
-      }
-      __syncthreads();
-      quit = uni(draw.quit);
-    }
-    if (quit) {
+    // the iteration before is over (first sweep), the sweeps are done (error pass)
+    const bool dropped = team_gate(
+        draw, it >= max_iter, sweep ? sw == 0 && it > 0 : true, threadIdx.x == 0,
+        [](int x) { return uni(x); },
+        [&]() {
+          const words_t word = &words[sweep ? kTeamState : kTeamSwept];
+          const int need = sweep ? it : td.R * (it + 1);
+          TPatience wait;
+          while (ld_dev(word) < need)
+            if (wait.over(words)) break;
+          return gone(words);
+        },
+        []() { __syncthreads(); });
+    if (dropped) {
       team = -1;
       __syncthreads();
       continue;
@@ -1132,8 +1125,8 @@ __global__ void __launch_bounds__(kTW * 64, WIDE ? 2 : 4)
         }
       }
     }
+    if (threadIdx.x == 0 && draw.quit) team = -1;
     __syncthreads();
-    team = draw.quit ? -1 : draw.team;
   }
 }
 
