@@ -69,12 +69,10 @@ __device__ __forceinline__ T fast2(T a, T b, T f, T h) {
   return d >= fh ? one : two;
 }
 
-constexpr int kSpin2 = 1 << 20;
-
 }  // namespace
 
 // MEM: the travel times stay in memory.  Reports fault = 2 (nothing done) if
-// the slowness is not tame.
+// the slowness is not tame, 1 if a wait ran out; u is then to be solved anew.
 template <typename T, bool MEM>
 __global__ void __launch_bounds__(1024) fwd2_band_kernel(Event2Desc ev, int max_iter) {
   __shared__ __attribute__((aligned(16))) char store[MEM ? 16 : kFwd2Lds];
@@ -209,16 +207,27 @@ __global__ void __launch_bounds__(1024) fwd2_band_kernel(Event2Desc ev, int max_
         }
         return r;
       };
-      // (bounded: every count is reached, as a wave waits only for earlier steps
-      // in the order (sweep, band); past the bound a fault is reported)
+      // Every count is reached, as a wave waits only for earlier steps in the order
+      // (sweep, band); how long it takes grows with the grid (a sweep that flips the
+      // long axis waits for all of the one before it).  So the bound is on the time
+      // in which no count of the workgroup moves; past it a fault is reported.
       int safe = -2;
       auto wait = [&](int v) {
+        int seen = -1;
+        uint64_t t0 = 0;
         for (int spin = 0; (safe = allowed()) < v; ++spin) {
           if (uni2(ld_lds(&flag[1]))) {
             safe = inf_v;
             break;
           }
-          if (spin > kSpin2) st_lds(&flag[1], 1);
+          if ((spin & 1023) == 1023) {
+            const int c = ld_lds(&prog[p >> 4][p & 15]);
+            const bool moved = __builtin_amdgcn_ballot_w64(c != seen) != 0;
+            const uint64_t now = wall_clock64();
+            seen = c;
+            t0 = moved ? now : t0;
+            if (now - t0 > kTeamPatience) st_lds(&flag[1], 1);
+          }
           __builtin_amdgcn_s_sleep(1);
         }
         fence2();
@@ -308,6 +317,8 @@ __global__ void __launch_bounds__(1024) fwd2_band_kernel(Event2Desc ev, int max_
       if (p == 0) st_lds(&prog[sw][w], V);
     }
     __syncthreads();
+    // a wait ran out: over (nothing is written to the flag until the next sweeps)
+    if (uni2(ld_lds(&flag[1]))) break;
     if constexpr (!MEM) {
       for (int q = threadIdx.x; q < N; q += nt) {
         const int j = q / m1, i = q - j * m1;
