@@ -175,6 +175,8 @@ def lib():
     L.adt_tune_save.restype = _i32
     L.adt_tune_load.argtypes = [ctypes.c_char_p]
     L.adt_tune_load.restype = _i32
+    L.adt_selftest_forward.argtypes = [_p, _i32, _i32, _i32, _i32, _p, _p, _p, _p]
+    L.adt_selftest_forward.restype = _i32
     L.adt_version.restype = ctypes.c_char_p
     L.adt_last_error.restype = ctypes.c_char_p
     _lib = L

@@ -602,3 +602,43 @@ def selftest_arith(op: int, a, b=None):
             _stream())
     L.check(rc, "selftest_arith")
     return out
+
+
+FORMS = ("stream", "one", "team", "wide")
+
+
+def selftest_forward_forms(shapes, dtype="float64", hs=None, compute_f64=False):
+    """The forward kernel that a batch of boxes takes under the present settings,
+    per event: "stream" or "one" (one workgroup), "team" or "wide" (several).
+    Nothing runs; no device is needed."""
+    n = len(shapes)
+    tab = (L.AdtEvent3d * n)()
+    for e, s in enumerate(shapes):
+        ev = tab[e]
+        ev.m, ev.n, ev.l = (int(x) for x in s)
+        ev.h = 1.0 if hs is None else float(hs[e])
+        ev.u0 = ev.f = ev.u = ctypes.addressof(tab)  # (not looked at)
+    forms, left = (ctypes.c_int32 * n)(), (ctypes.c_int32 * n)()
+    rc = L.lib().adt_selftest_forward(ctypes.byref(tab), n, _flags(True, None, compute_f64),
+                                      _dtype_code(dtype), -1, forms, left, None, None)
+    L.check(rc, "selftest_forward")
+    return [FORMS[k] for k in forms]
+
+
+def selftest_forward(u0s, fs, hs, tols, form=None, us=None, compute_f64=False):
+    """eikonal3d_batched's forward on the kernels named by ``form`` (None: the
+    library's choice).  Returns dict(u, info, form, left): what each event ran on,
+    and 1 or 2 where several workgroups left it to one."""
+    torch = _torch()
+    n = len(fs)
+    if us is None:
+        us = [torch.empty_like(f) for f in fs]
+    tab, dtype = _event_table(u0s, fs, hs, tols, None, us, None, None)
+    infos = (L.AdtInfo * n)()
+    forms, left = (ctypes.c_int32 * n)(), (ctypes.c_int32 * n)()
+    rc = L.lib().adt_selftest_forward(ctypes.byref(tab), n, _flags(True, None, compute_f64),
+                                      _dtype_code(dtype), -1 if form is None else FORMS.index(form),
+                                      forms, left, infos, _stream())
+    L.check(rc, "selftest_forward")
+    return {"u": us, "info": [_checked(i.as_dict()) for i in infos],
+            "form": [FORMS[k] for k in forms], "left": list(left)}

@@ -507,6 +507,8 @@ struct TeamPlan {
 // storage 28, 18, 12.2; 256 uneven ones 47, 49, 26; 200 of 200x200x80 241, 347,
 // 141; 256 of 128x128x64 FP64 48, 136, 49.
 enum class Forward { kOne, kTeam, kWide };
+static_assert((int)Forward::kTeam == ADT_FORM_TEAM - ADT_FORM_ONE &&
+                  (int)Forward::kWide == ADT_FORM_WIDE - ADT_FORM_ONE, "forms");
 template <typename T>
 Forward choose_forward(const std::vector<adt::EventDesc>& descs) {
   const int cus = device_cus(), xcds = std::max(1, cus / 32), nev = (int)descs.size();
@@ -1427,8 +1429,9 @@ struct BatchPlan {
   }
   // Routes the forward to fwd3_team_kernel where the settings leave the
   // choice open and the events are too few or too uneven for one workgroup
-  // each; after order_largest_first (the plan's indices are final).
-  void plan_teams(int flags, const adt_tune& tn) {
+  // each; after order_largest_first (the plan's indices are final).  `form`
+  // (ADT_FORM_*): a test's choice in place of the library's.
+  void plan_teams(int flags, const adt_tune& tn, int form = -1) {
     if (!(flags & ADT_FORWARD) || descs.empty()) return;
     if (fused(flags, mix, tn)) return;
     std::vector<int> use;
@@ -1436,9 +1439,19 @@ struct BatchPlan {
       if (!descs[e].pad || !TeamPlan::fits<T>(descs[e])) return;
       use.push_back((int)e);
     }
-    const Forward how = choose_forward<T>(descs);
+    const Forward how = form >= 0 ? (Forward)(form - ADT_FORM_ONE) : choose_forward<T>(descs);
     if (how == Forward::kOne) return;
     ws_bytes = team.build<T>(descs, use, how == Forward::kWide, ws_bytes);
+  }
+  // The caller's index of an event (base: nullptr before bind()).
+  int index_of(const adt::EventDesc& d, const char* base) const {
+    return (int)(((const char*)d.info - base - off_info) / sizeof(adt_info));
+  }
+  // Each event's forward kernel (ADT_FORM_*), before bind().
+  void forms(int32_t* out) const {
+    for (const adt::EventDesc& d : descs)
+      out[index_of(d, nullptr)] = d.team_words ? (team.wide ? ADT_FORM_WIDE : ADT_FORM_TEAM)
+                                  : d.fwd_diag ? ADT_FORM_ONE : ADT_FORM_STREAM;
   }
   void bind(char* base) {
     team.bind(base, descs);
@@ -1519,9 +1532,17 @@ int launch_batch(const BatchPlan<T>& plan, char* base, int nev, int flags, const
   return ADT_OK;
 }
 
+// A test's view of a batched call (adt_selftest_forward).
+struct ForwardProbe {
+  int form;        // ADT_FORM_* to run, or -1: the library's choice
+  int32_t* forms;  // out: the form of each event
+  int32_t* left;   // out: an event's abort word (0: the team kernel solved it)
+  bool plan_only;
+};
+
 template <typename T>
 int batched_impl(const adt_event3d* ev, int nev, int flags, adt_info* infos, void* stream,
-                 const MisfitArgs* mis = nullptr) {
+                 const MisfitArgs* mis = nullptr, const ForwardProbe* probe = nullptr) {
   if (!(flags & (ADT_FORWARD | ADT_ADJOINT))) return fail(ADT_EINVAL, "batched: no ADT_FORWARD/ADT_ADJOINT flag");
   if (flags & ADT_HOST_POINTERS) return fail(ADT_EINVAL, "batched: device pointers only");
   if (mis && !((flags & ADT_FORWARD) && (flags & ADT_ADJOINT)))
@@ -1535,7 +1556,11 @@ int batched_impl(const adt_event3d* ev, int nev, int flags, adt_info* infos, voi
   if (mis && (rc = plan.attach_misfit(ev, nev, mis))) return rc;
   if (nev == 0) return ADT_OK;
   if (tn.order) plan.order_largest_first();
-  plan.plan_teams(flags, tn);
+  plan.plan_teams(flags, tn, probe ? probe->form : -1);
+  if (probe) {
+    plan.forms(probe->forms);
+    if (probe->plan_only) return ADT_OK;
+  }
   DevBuf ws;
   if ((rc = ws.alloc(plan.ws_bytes, s))) return rc;
   plan.bind((char*)ws.p);
@@ -1556,6 +1581,11 @@ int batched_impl(const adt_event3d* ev, int nev, int flags, adt_info* infos, voi
       if (infos[e].fault)
         return fail(ADT_EHIP, "batched: wave synchronisation timed out in event " + std::to_string(e));
   }
+  if (probe)
+    for (const adt::EventDesc& d : plan.descs)
+      if (d.team_words)
+        ADT_HIP(hipMemcpy(&probe->left[plan.index_of(d, base)], d.team_words + adt::kTeamAbort,
+                          sizeof(int32_t), hipMemcpyDeviceToHost));
   return ADT_OK;
 }
 
@@ -2541,6 +2571,18 @@ int adt_sum_arrays_f64(const double* const* arrays, int32_t narr, int64_t N, dou
 int adt_sum_arrays_f32(const float* const* arrays, int32_t narr, int64_t N, float* out,
                        void* stream) {
   return sum_arrays_impl<float>(arrays, narr, N, out, stream);
+}
+
+int adt_selftest_forward(const adt_event3d* events, int32_t nev, int32_t flags, int32_t dtype,
+                         int32_t form, int32_t* forms, int32_t* left, adt_info* infos,
+                         void* stream) {
+  if (nev < 1 || !forms || !left || (dtype != 0 && dtype != 1) ||
+      (form != -1 && (form < ADT_FORM_ONE || form > ADT_FORM_WIDE)))
+    return fail(ADT_EINVAL, "selftest: bad arguments");
+  for (int e = 0; e < nev; ++e) left[e] = 0;
+  const ForwardProbe p{form, forms, left, infos == nullptr};
+  return dtype == 0 ? batched_impl<double>(events, nev, flags, infos, stream, nullptr, &p)
+                    : batched_impl<float>(events, nev, flags, infos, stream, nullptr, &p);
 }
 
 int adt_selftest_arith_f64(int32_t op, const double* a, const double* b, double* out, int64_t n,

@@ -411,6 +411,21 @@ int adt_selftest_arith_f64(int32_t op, const double *a, const double *b, double 
 int adt_selftest_arith_f32(int32_t op, const float *a, const float *b, float *out, int64_t n,
                            void *stream);
 
+/* ---- Diagnostics: the forward kernel of each event of a batched call.
+ * As adt_eikonal3d_batched_* with the same events and flags, but with `form`
+ * (ADT_FORM_ONE, _TEAM or _WIDE) in place of the library's choice where the
+ * settings leave it open, or the library's (-1).  forms[nev]: what ran;
+ * left[nev]: 0, or why several workgroups left the event to one (1: values
+ * that their local solve does not cover, 2: a wait ran out).  With infos NULL
+ * only the choice is made: nothing runs and no device is needed. */
+#define ADT_FORM_STREAM 0 /* one workgroup, k-streaming */
+#define ADT_FORM_ONE 1    /* one workgroup, diagonals */
+#define ADT_FORM_TEAM 2   /* several workgroups, 16 bytes of k per lane */
+#define ADT_FORM_WIDE 3   /* several workgroups, eight nodes of k per lane */
+int adt_selftest_forward(const adt_event3d *events, int32_t nev, int32_t flags, int32_t dtype,
+                         int32_t form, int32_t *forms, int32_t *left, adt_info *infos,
+                         void *stream);
+
 #ifdef __cplusplus
 }
 #endif
