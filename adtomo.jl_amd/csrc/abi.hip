@@ -8,10 +8,12 @@
 #include <cstdio>
 #include <cstring>
 #include <algorithm>
+#include <functional>
 #include <limits>
 #include <list>
 #include <map>
 #include <mutex>
+#include <queue>
 #include <set>
 #include <string>
 #include <type_traits>
@@ -431,6 +433,20 @@ struct TeamPlan {
     t.E = (int)std::max<int64_t>(1, std::min<int64_t>(32, N / 8192));
     return t;
   }
+  // Workgroups of a launch over nt events of at most maxR regions: up to 4 per
+  // compute unit, 2 of the wide form (the kernels' occupancy; 3 of the wide form
+  // in FP64 need spills and are slower: 60 against 49 ms on 256 events of
+  // 128x128x64); an event has work for about 2.5 sweeps' regions at a time.
+  struct Groups {
+    int xcds, slots, size, per_xcd;  // slots: workgroups that an XCD holds at a time
+  };
+  static Groups groups(int nt, int64_t maxR, bool wide) {
+    const int cus = device_cus(), xcds = std::max(1, cus / 32);
+    const int slots = (wide ? 2 : 4) * cus / xcds;
+    const int here = std::min((nt + xcds - 1) / xcds, slots);  // events per XCD at a time
+    const int size = (int)std::max<int64_t>(1, std::min<int64_t>(slots / here, (5 * maxR + 1) / 2 + 1));
+    return Groups{xcds, slots, size, std::min(slots, here * size)};
+  }
   // Lays out the words of the events `use` (indices into evs) from byte
   // offset `off` on; returns the end.
   template <typename T>
@@ -455,16 +471,9 @@ struct TeamPlan {
       descs.push_back(t);
     }
     zero_bytes = off - off_zero;
-    // workgroups: up to 4 per compute unit, 2 of the wide form (the kernels'
-    // occupancy; 3 of the wide form with spills are slower: 60 against 49 ms on 256
-    // events of 128x128x64); an event
-    // has work for about 2.5 sweeps' regions at a time
-    const int cus = device_cus(), xcds = std::max(1, cus / 32);
-    const int slots = (wide ? 2 : 4) * cus / xcds;
-    const int here = (nt + xcds - 1) / xcds;  // events per XCD at a time
-    per_group = (int)std::max<int64_t>(1, std::min<int64_t>(slots / std::min(here, slots),
-                                                          (5 * maxR + 1) / 2 + 1));
-    grid = xcds * std::min(slots, here * per_group);
+    const Groups g = groups(nt, maxR, wide);
+    per_group = g.size;
+    grid = g.xcds * g.per_xcd;
     return off;
   }
   void bind(char* base, std::vector<adt::EventDesc>& evs) {
@@ -491,21 +500,69 @@ struct TeamPlan {
   }
 };
 
-// Which forward kernel suits these events?  Each one's time for one iteration,
-// from the steps it takes (microseconds a step as measured on an MI355X; the
-// iteration counts are the same):
-//   one workgroup per event: bands * N_b + H + 6 steps per sweep and k chunk,
-//     2.4 us + 0.27 us per node of a lane, half as much again where every CU has
-//     an event (they share the memory);
-//   several: an event alone takes 4 (M_a + N_b) + 30 slabs + 80 steps (its
-//     sweeps overlap), many are bound by the wave steps of all of them, on the
-//     CUs of the XCDs that have an event.  With 16 bytes of k per lane 1.1 us a
-//     step and 0.44 us per CU for each wave step (accesses to the L2, 16 bytes
-//     each); with eight nodes 2.6 us and 0.72 us (the local solves).
-// Forward of one workgroup, 16 bytes, eight nodes, in ms: one event of 128x128x64
-// FP64 28, 5.5, 10; 16 of 101x90x47 27, 5.0, 8.1; 64 of 128x128x64 with FP32
-// storage 28, 18, 12.2; 256 uneven ones 47, 49, 26; 200 of 200x200x80 241, 347,
-// 141; 256 of 128x128x64 FP64 48, 136, 49.
+// The forms' times for one iteration, in microseconds as measured on an MI355X
+// with 20 iterations of every event (80 sets of events in each precision).
+
+// One workgroup, an event alone: its steps, in chains of sweeps where all of k is
+// one chunk (20 us to begin a chain), 4.3 us a step with eight nodes a lane (FP32
+// 3.8), else 3.1 + 0.34 per node.
+template <typename T>
+double one_workgroup_us(const adt::EventDesc& d) {
+  const adt::TeamDesc t = TeamPlan::geometry<T>(d, false);
+  const int Nb = std::max(d.m, d.n);
+  constexpr int kChunk = 8 * kSegsMax;
+  // of an iteration's seven turns three flip a, three flip b
+  const int chains = d.l > kChunk ? 8 : 8 - 3 * (Nb >= t.H + 3) - 3 * (t.bands >= 2);
+  const double steps = 8.0 * t.bands * Nb + chains * (t.H - 1);
+  double us = 0;
+  for (int c = 0; c < d.l; c += kChunk) {
+    const int lw = (std::min(d.l - c, kChunk) + kSegsMax - 1) / kSegsMax;
+    us += chains * 20 + steps * (lw < 8 ? 3.1 + 0.34 * lw : sizeof(T) == 8 ? 4.3 : 3.8);
+  }
+  return us;
+}
+// One workgroup each: handed out largest first, or, where that is more, their
+// accesses: 64 bytes of u, f and u again for eight nodes (in FP32 as well), 1.6 times
+// as many where columns do not begin on them, at the rate of a large copy.
+template <typename T>
+double one_workgroup_each_us(const std::vector<adt::EventDesc>& descs, int cus) {
+  std::vector<double> us;
+  double mem = 0, last = 0;
+  for (const adt::EventDesc& d : descs) {
+    us.push_back(one_workgroup_us<T>(d));
+    mem += 8 * 3 * 8.0 * d.m * d.n * d.l * (d.l % 8 ? 1.6 : 1) / 4.92e6;
+  }
+  std::sort(us.begin(), us.end(), std::greater<double>());
+  std::priority_queue<double, std::vector<double>, std::greater<double>> ends;
+  for (double at : us) {
+    if ((int)ends.size() == cus) {
+      at += ends.top();
+      ends.pop();
+    }
+    ends.push(at);
+    last = std::max(last, at);
+  }
+  return std::cbrt(last * last * last + mem * mem * mem);
+}
+
+// Which forward kernel suits these events?  Several workgroups: an event alone
+// takes 4 (M_a + N_b) + 30 slabs + 80 steps (its sweeps overlap), many are bound by
+// the wave steps of all of them, on the CUs of the XCDs that have an event.  With
+// 16 bytes of k per lane 1.1 us a step and 0.44 us per CU for each wave step
+// (accesses to the L2, 16 bytes each); with eight nodes 2.6 us and 0.36 us + 0.40
+// for a step's worth of nodes (the local solves; 0.875 of it in FP32, 1.25 where
+// columns do not begin on 64 bytes), and more where the groups do not fill the
+// XCD: an event has slots / (events of an XCD) workgroups, rounded down, each
+// faster by a third of what the others leave idle.
+// How many iterations there are differs by event (2 and 3, or 3 and 4): one
+// workgroup each takes as long as the event with the most, the others as the mean.
+// So several workgroups are taken up to 1.05 times the first form's time.
+// One workgroup, 16 bytes, eight nodes, ms of 20 iterations in FP64: 1 event of
+// 128x128x64 185, 37, 63; 64 190, 220, 98; 160 211, 553, 198; 176 216, 608, 251; 208
+// 227, 714, 273; 256 250, 897, 297; 250 of 60x128x64 130, 394, 140; 16 of 101x90x47
+// 177, 31, 53; 256 222, 447, 204; 200 of 200x200x80 1237, 2196, 878; 256 uneven
+// ones up to 128x128x64 314, 426, 202; with FP32 storage 160 of 128x128x64 192,
+// 280, 174; 208 213, 362, 239.
 enum class Forward { kOne, kTeam, kWide };
 static_assert((int)Forward::kTeam == ADT_FORM_TEAM - ADT_FORM_ONE &&
                   (int)Forward::kWide == ADT_FORM_WIDE - ADT_FORM_ONE, "forms");
@@ -513,27 +570,26 @@ template <typename T>
 Forward choose_forward(const std::vector<adt::EventDesc>& descs) {
   const int cus = device_cus(), xcds = std::max(1, cus / 32), nev = (int)descs.size();
   const double used = (double)cus * std::min(1.0, (double)nev / xcds);
-  double dmax = 0, dsum = 0, tmax[2] = {0, 0}, tsum[2] = {0, 0};
+  double tmax[2] = {0, 0}, tsum[2] = {0, 0};
+  int64_t maxR = 1;
   for (const adt::EventDesc& d : descs) {
     const double Ma = std::min(d.m, d.n), Nb = std::max(d.m, d.n);
-    double one = 0;
     for (int w = 0; w < 2; ++w) {
       const adt::TeamDesc t = TeamPlan::geometry<T>(d, w == 1);
-      const double segs = std::ceil(d.l / (w ? 8.0 : 16.0 / sizeof(T)));
+      const double segs = std::ceil(d.l / (w ? 8.0 : 16.0 / sizeof(T))), steps = Nb + t.H - 1;
+      const double wide = (0.36 * steps + 0.40 * Nb * t.H / 64) * (sizeof(T) == 8 ? 1 : 0.875) *
+                          (d.l % 8 ? 1.25 : 1);
       tmax[w] = std::max(tmax[w], (4 * (Ma + Nb) + 30 * t.ns + 80) * (w ? 2.6 : 1.1));
-      tsum[w] += 8 * t.bands * (Nb + t.H - 1) * segs * (w ? 0.72 : 0.44);
-      if (w) continue;
-      for (int c = 0; c < d.l; c += 8 * kSegsMax) {
-        const int lw = (std::min(d.l - c, 8 * kSegsMax) + kSegsMax - 1) / kSegsMax;
-        one += 8 * (t.bands * Nb + t.H + 6) * (2.4 + 0.27 * lw);
-      }
+      tsum[w] += 8 * t.bands * segs * (w ? wide : 0.44 * steps);
+      if (w) maxR = std::max<int64_t>(maxR, t.R);
     }
-    dmax = std::max(dmax, one);
-    dsum += one;
   }
-  const double td = std::max(dmax * (1 + 0.5 * std::min(1.0, (double)nev / cus)), 1.5 * dsum / cus);
-  const double t0 = std::max(tmax[0], tsum[0] / used), t1 = std::max(tmax[1], tsum[1] / used);
-  if (std::min(t0, t1) >= 0.9 * td) return Forward::kOne;
+  const TeamPlan::Groups g = TeamPlan::groups(nev, maxR, true);
+  // (more workgroups than an event has work for: none of them is missed)
+  const double idle = g.size == (5 * maxR + 1) / 2 + 1 ? 1 : 2 / 3.0 + g.slots / (3.0 * g.per_xcd);
+  const double td = one_workgroup_each_us<T>(descs, cus);
+  const double t0 = std::max(tmax[0], tsum[0] / used), t1 = std::max(tmax[1], tsum[1] / used * idle);
+  if (std::min(t0, t1) >= 1.05 * td) return Forward::kOne;
   return t0 <= t1 ? Forward::kTeam : Forward::kWide;
 }
 
