@@ -529,6 +529,7 @@ double one_workgroup_each_us(const std::vector<adt::EventDesc>& descs, int cus) 
   std::vector<double> us;
   double mem = 0, last = 0;
   for (const adt::EventDesc& d : descs) {
+    if (!d.fwd_diag) continue;
     us.push_back(one_workgroup_us<T>(d));
     mem += 8 * 3 * 8.0 * d.m * d.n * d.l * (d.l % 8 ? 1.6 : 1) / 4.92e6;
   }
@@ -557,6 +558,8 @@ double one_workgroup_each_us(const std::vector<adt::EventDesc>& descs, int cus) 
 // How many iterations there are differs by event (2 and 3, or 3 and 4): one
 // workgroup each takes as long as the event with the most, the others as the mean.
 // So several workgroups are taken up to 1.05 times the first form's time.
+// Events that are not in `use` stay with one workgroup each and run behind the
+// others: their time is added to that of several workgroups.
 // One workgroup, 16 bytes, eight nodes, ms of 20 iterations in FP64: 1 event of
 // 128x128x64 185, 37, 63; 64 190, 220, 98; 160 211, 553, 198; 176 216, 608, 251; 208
 // 227, 714, 273; 256 250, 897, 297; 250 of 60x128x64 130, 394, 140; 16 of 101x90x47
@@ -567,12 +570,15 @@ enum class Forward { kOne, kTeam, kWide };
 static_assert((int)Forward::kTeam == ADT_FORM_TEAM - ADT_FORM_ONE &&
                   (int)Forward::kWide == ADT_FORM_WIDE - ADT_FORM_ONE, "forms");
 template <typename T>
-Forward choose_forward(const std::vector<adt::EventDesc>& descs) {
-  const int cus = device_cus(), xcds = std::max(1, cus / 32), nev = (int)descs.size();
+Forward choose_forward(const std::vector<adt::EventDesc>& descs, const std::vector<int>& use) {
+  const int cus = device_cus(), xcds = std::max(1, cus / 32), nev = (int)use.size();
   const double used = (double)cus * std::min(1.0, (double)nev / xcds);
   double tmax[2] = {0, 0}, tsum[2] = {0, 0};
   int64_t maxR = 1;
-  for (const adt::EventDesc& d : descs) {
+  std::vector<adt::EventDesc> rest = descs;
+  for (const int e : use) {
+    const adt::EventDesc& d = descs[e];
+    rest[e].fwd_diag = 0;
     const double Ma = std::min(d.m, d.n), Nb = std::max(d.m, d.n);
     for (int w = 0; w < 2; ++w) {
       const adt::TeamDesc t = TeamPlan::geometry<T>(d, w == 1);
@@ -589,7 +595,7 @@ Forward choose_forward(const std::vector<adt::EventDesc>& descs) {
   const double idle = g.size == (5 * maxR + 1) / 2 + 1 ? 1 : 2 / 3.0 + g.slots / (3.0 * g.per_xcd);
   const double td = one_workgroup_each_us<T>(descs, cus);
   const double t0 = std::max(tmax[0], tsum[0] / used), t1 = std::max(tmax[1], tsum[1] / used * idle);
-  if (std::min(t0, t1) >= 1.05 * td) return Forward::kOne;
+  if (std::min(t0, t1) + one_workgroup_each_us<T>(rest, cus) >= 1.05 * td) return Forward::kOne;
   return t0 <= t1 ? Forward::kTeam : Forward::kWide;
 }
 
@@ -634,7 +640,7 @@ int fwd3_impl(const T* u0, const T* f, T h, int64_t m, int64_t n, int64_t l, T t
   const size_t off_info = ((bytes + 255) / 256) * 256;
   const size_t off_desc = off_info + ((sizeof(adt_info) + 255) / 256) * 256;
   size_t end = off_desc + 256;
-  const Forward how = snap.leaves_open(m, n, l) && TeamPlan::fits<T>(d) ? choose_forward<T>(ds) : Forward::kOne;
+  const Forward how = snap.leaves_open(m, n, l) && TeamPlan::fits<T>(d) ? choose_forward<T>(ds, {0}) : Forward::kOne;
   if (how != Forward::kOne) end = team.build<T>(ds, {0}, how == Forward::kWide, end);
   DevBuf ws;
   if ((rc = ws.alloc(end, s))) return rc;
@@ -1483,19 +1489,18 @@ struct BatchPlan {
       return (int64_t)a.m * a.n * a.l > (int64_t)b.m * b.n * b.l;
     });
   }
-  // Routes the forward to fwd3_team_kernel where the settings leave the
-  // choice open and the events are too few or too uneven for one workgroup
-  // each; after order_largest_first (the plan's indices are final).  `form`
-  // (ADT_FORM_*): a test's choice in place of the library's.
+  // Routes the forward of the events whose settings leave the choice open to
+  // fwd3_team_kernel where they are too few or too uneven for one workgroup each;
+  // after order_largest_first (the plan's indices are final).  The others keep
+  // their kernel.  `form` (ADT_FORM_*): a choice in place of the library's.
   void plan_teams(int flags, const adt_tune& tn, int form = -1) {
     if (!(flags & ADT_FORWARD) || descs.empty()) return;
     if (fused(flags, mix, tn)) return;
     std::vector<int> use;
-    for (size_t e = 0; e < descs.size(); ++e) {
-      if (!descs[e].pad || !TeamPlan::fits<T>(descs[e])) return;
-      use.push_back((int)e);
-    }
-    const Forward how = form >= 0 ? (Forward)(form - ADT_FORM_ONE) : choose_forward<T>(descs);
+    for (size_t e = 0; e < descs.size(); ++e)
+      if (descs[e].pad && TeamPlan::fits<T>(descs[e])) use.push_back((int)e);
+    if (use.empty()) return;
+    const Forward how = form >= 0 ? (Forward)(form - ADT_FORM_ONE) : choose_forward<T>(descs, use);
     if (how == Forward::kOne) return;
     ws_bytes = team.build<T>(descs, use, how == Forward::kWide, ws_bytes);
   }
@@ -1839,7 +1844,7 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
   bool team_ok = false;
   if (flags & ADT_FORWARD) {
     std::vector<adt::EventDesc> ds(nev);
-    team_ok = true;
+    std::vector<int> use;
     for (int e = 0; e < nev; ++e) {
       ds[e] = adt::EventDesc{};
       ds[e].m = (int)ev[e].m;
@@ -1847,9 +1852,9 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
       ds[e].l = (int)ev[e].l;
       ds[e].h = ev[e].h;
       ds[e].fwd_diag = 1;
-      team_ok = team_ok && TeamPlan::fits<T>(ds[e]);
+      if (TeamPlan::fits<T>(ds[e])) use.push_back(e);
     }
-    team_ok = team_ok && choose_forward<T>(ds) != Forward::kOne;
+    team_ok = !use.empty() && choose_forward<T>(ds, use) != Forward::kOne;
   }
   std::map<ClassKey, adt_tune> classes = cur.classes;
   std::set<ClassKey> open = cur.open;
