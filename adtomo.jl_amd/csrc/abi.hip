@@ -1812,15 +1812,15 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
     return fail(ADT_EHIP, std::string("autotune: hipEventCreate: ") + hipGetErrorString(he));
   }
   // mean time of `reps` launches of `evs` under snapshot `sn` with flags
-  // `fl`, after one untimed launch
+  // `fl`, after one untimed launch; form: see plan_teams
   auto time_set = [&](const std::vector<adt_event3d>& evs, const TuneSnap& sn, int fl,
-                      float* ms) -> int {
+                      float* ms, int form = -1) -> int {
     const int n = (int)evs.size();
     BatchPlan<T> plan;
     int r = plan.build(evs.data(), n, fl, sn);
     if (r) return r;
     if (sn.global.order) plan.order_largest_first();
-    plan.plan_teams(fl, sn.global);
+    plan.plan_teams(fl, sn.global, form);
     DevBuf ws;
     if ((r = ws.alloc(plan.ws_bytes, s))) return r;
     plan.bind((char*)ws.p);
@@ -1839,9 +1839,8 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
     return ADT_OK;
   };
   int rc = ADT_OK;
-  // several workgroups per event (fwd_segs 0) where that is the library's
-  // choice for all of the events
-  bool team_ok = false;
+  // the library's choice for all of the events
+  Forward how = Forward::kOne;
   if (flags & ADT_FORWARD) {
     std::vector<adt::EventDesc> ds(nev);
     std::vector<int> use;
@@ -1854,7 +1853,7 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
       ds[e].fwd_diag = 1;
       if (TeamPlan::fits<T>(ds[e])) use.push_back(e);
     }
-    team_ok = !use.empty() && choose_forward<T>(ds, use) != Forward::kOne;
+    if (!use.empty()) how = choose_forward<T>(ds, use);
   }
   std::map<ClassKey, adt_tune> classes = cur.classes;
   std::set<ClassKey> open = cur.open;
@@ -1894,19 +1893,19 @@ int autotune_impl(const adt_event3d* ev, int nev, int flags, int reps, adt_tune*
         }
       }
       if (rc) break;
+      // The class is fixed where several workgroups, as all of the events would
+      // take them, were slower on its own; where they take one each, nothing was
+      // learnt of several, and launches of fewer events may still choose them.
       open.erase(it->first);
-      if (team_ok) {
-        TuneSnap t1 = sc;
-        t1.classes.clear();
-        t1.open.clear();
-        t1.global.diag_max_l = adt::kDiagAll;
-        t1.global.fwd_segs = 0;
+      if (sc.global.diag_max_l == adt::kDiagAll) {
         float ms = 0.f;
-        if ((rc = time_set(evs, t1, ADT_FORWARD | fmix, &ms))) break;
-        if (ms < fbest && sc.global.diag_max_l == adt::kDiagAll) {
-          fbest = ms;
-          open.insert(it->first);
+        if (how != Forward::kOne) {
+          TuneSnap t1 = sc;
+          t1.global.fwd_segs = 0;
+          if ((rc = time_set(evs, t1, ADT_FORWARD | fmix, &ms, ADT_FORM_ONE + (int)how))) break;
         }
+        if (ms < fbest) open.insert(it->first);
+        if (how != Forward::kOne) fbest = std::min(fbest, ms);
       }
     }
     if (flags & ADT_ADJOINT) {
