@@ -18,12 +18,14 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 import numpy as np
 
 from . import _lib as L
 
 last_info: dict = {}
+FAULT_SOLVED = 2  # adt_info.fault: solved anew after a wait that timed out
 
 
 def _torch():
@@ -46,8 +48,11 @@ def _stream():
 
 def _checked(info: dict) -> dict:
     """Raises if a kernel reported an internal fault for this event (a
-    bounded wait between its waves timed out; its results are invalid)."""
-    if info.get("fault"):
+    bounded wait between its waves timed out; its results are invalid), and
+    warns if another kernel then solved it."""
+    if info.get("fault") == FAULT_SOLVED:
+        warnings.warn("wave synchronisation timed out in an event's forward; it was solved anew")
+    elif info.get("fault"):
         raise L.AdtError("kernel fault reported for an event (wave synchronisation timed out)")
     return info
 
@@ -625,17 +630,18 @@ def selftest_forward_forms(shapes, dtype="float64", hs=None, compute_f64=False):
     return [FORMS[k] for k in forms]
 
 
-def selftest_forward(u0s, fs, hs, tols, form=None, us=None, compute_f64=False):
+def selftest_forward(u0s, fs, hs, tols, form=None, us=None, compute_f64=False, left=None):
     """eikonal3d_batched's forward on the kernels named by ``form`` (None: the
     library's choice).  Returns dict(u, info, form, left): what each event ran on,
-    and 1 or 2 where several workgroups left it to one."""
+    and 1 or 2 where several workgroups left it to one (``left``: where they are
+    to, at once)."""
     torch = _torch()
     n = len(fs)
     if us is None:
         us = [torch.empty_like(f) for f in fs]
     tab, dtype = _event_table(u0s, fs, hs, tols, None, us, None, None)
     infos = (L.AdtInfo * n)()
-    forms, left = (ctypes.c_int32 * n)(), (ctypes.c_int32 * n)()
+    forms, left = (ctypes.c_int32 * n)(), (ctypes.c_int32 * n)(*(left or ()))
     rc = L.lib().adt_selftest_forward(ctypes.byref(tab), n, _flags(True, None, compute_f64),
                                       _dtype_code(dtype), -1 if form is None else FORMS.index(form),
                                       forms, left, infos, _stream())

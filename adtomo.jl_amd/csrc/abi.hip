@@ -670,7 +670,7 @@ int fwd3_impl(const T* u0, const T* f, T h, int64_t m, int64_t n, int64_t l, T t
   ADT_HIP(hipStreamSynchronize(s));
   if (verbose) print_verbose(hinf);
   if (info) *info = hinf;
-  if (hinf.fault) return fail(ADT_EHIP, "eikonal3d: wave synchronisation timed out in the kernel");
+  if (hinf.fault == ADT_FAULT) return fail(ADT_EHIP, "eikonal3d: wave synchronisation timed out in the kernel");
   return ADT_OK;
 }
 
@@ -751,7 +751,7 @@ int fwd3_noalloc_impl(const double* u0, const double* f, double h, int64_t m, in
   ADT_HIP(hipStreamSynchronize(s));
   if (verbose) print_verbose(hinf);
   if (info) *info = hinf;
-  if (hinf.fault) return fail(ADT_EHIP, "eikonal3d: wave synchronisation timed out in the kernel");
+  if (hinf.fault == ADT_FAULT) return fail(ADT_EHIP, "eikonal3d: wave synchronisation timed out in the kernel");
   return ADT_OK;
 }
 
@@ -863,7 +863,7 @@ int fwd2_impl(const T* f, int64_t m, int64_t n, int64_t srcx, int64_t srcy, T h,
   const int64_t rows = std::min(m, n) + 1, cols = std::max(m, n) + 1;
   const int waves = (int)((rows + 63) / 64);
   const int nt = 64 * (waves <= 8 ? 2 * waves : waves);
-  bool done = false;
+  bool done = false, late = false;
   if (waves <= 16 && N < (int64_t(1) << 28)) {
     const size_t lds = sizeof(T) * (size_t)(rows + 2) * (size_t)((cols + 3) & ~int64_t(1));
     if (lds <= (size_t)adt::kFwd2Lds)
@@ -873,8 +873,9 @@ int fwd2_impl(const T* f, int64_t m, int64_t n, int64_t srcx, int64_t srcy, T h,
     ADT_HIP(hipGetLastError());
     ADT_HIP(hipMemcpyAsync(&hinf, d.info, sizeof(adt_info), hipMemcpyDeviceToHost, s));
     ADT_HIP(hipStreamSynchronize(s));
-    // 2: slowness that its fast solve does not cover; 1: a wait ran out
+    // 2: slowness that its fast solve does not cover; ADT_FAULT: a wait ran out
     done = hinf.fault == 0;
+    late = hinf.fault == ADT_FAULT;
   }
   if (!done) {
     ADT_HIP(hipMemcpyAsync(base + a, &d, sizeof(d), hipMemcpyHostToDevice, s));
@@ -885,6 +886,7 @@ int fwd2_impl(const T* f, int64_t m, int64_t n, int64_t srcx, int64_t srcy, T h,
   }
   if (hp) ADT_HIP(hipMemcpyAsync(u, du, bytes, hipMemcpyDeviceToHost, s));
   ADT_HIP(hipStreamSynchronize(s));
+  if (late) hinf.fault = ADT_FAULT_SOLVED;
   if (!hinf.converged) fprintf(stderr, "ERROR: Eikonal does not converge!\n");
   if (info) *info = hinf;
   return ADT_OK;
@@ -1540,7 +1542,7 @@ struct BatchPlan {
 // event's adjoint traversal likewise.  tn: the launch-wide fields.
 template <typename T>
 int launch_batch(const BatchPlan<T>& plan, char* base, int nev, int flags, const adt_tune& tn,
-                 hipStream_t s, const MisfitRun& mr = MisfitRun{}) {
+                 hipStream_t s, const MisfitRun& mr = MisfitRun{}, const int32_t* left = nullptr) {
   if (nev == 0) return ADT_OK;
   const adt::EventDesc* ddesc = (const adt::EventDesc*)(base + plan.off_desc);
   const KernelMix& km = plan.mix;
@@ -1564,6 +1566,10 @@ int launch_batch(const BatchPlan<T>& plan, char* base, int nev, int flags, const
   }
   if (flags & ADT_FORWARD) {
     if (team.on()) {
+      for (const adt::EventDesc& d : plan.descs)
+        if (left && d.team_words)
+          ADT_HIP(hipMemcpyAsync((int*)d.team_words + adt::kTeamAbort, &left[plan.index_of(d, base)],
+                                 sizeof(int32_t), hipMemcpyHostToDevice, s));
       team.launch<T>(mix, ddesc, base, s);
       ADT_HIP(hipGetLastError());
     }
@@ -1597,7 +1603,7 @@ int launch_batch(const BatchPlan<T>& plan, char* base, int nev, int flags, const
 struct ForwardProbe {
   int form;        // ADT_FORM_* to run, or -1: the library's choice
   int32_t* forms;  // out: the form of each event
-  int32_t* left;   // out: an event's abort word (0: the team kernel solved it)
+  int32_t* left;   // an event's abort word; in: what the launch finds in it
   bool plan_only;
 };
 
@@ -1630,7 +1636,9 @@ int batched_impl(const adt_event3d* ev, int nev, int flags, adt_info* infos, voi
                          hipMemcpyHostToDevice, s));
   if ((rc = plan.upload_teams(base, s))) return rc;
   if ((rc = plan.upload_misfit(base, nev, s))) return rc;
-  if ((rc = launch_batch<T>(plan, base, nev, flags, tn, s, plan.misfit_run(base)))) return rc;
+  if ((rc = launch_batch<T>(plan, base, nev, flags, tn, s, plan.misfit_run(base),
+                            probe ? probe->left : nullptr)))
+    return rc;
   // the misfit table and coordinates were copied from the caller's host
   // memory: wait before returning
   if (mis && !infos) ADT_HIP(hipStreamSynchronize(s));
@@ -1639,7 +1647,7 @@ int batched_impl(const adt_event3d* ev, int nev, int flags, adt_info* infos, voi
                            hipMemcpyDeviceToHost, s));
     ADT_HIP(hipStreamSynchronize(s));
     for (int e = 0; e < nev; ++e)
-      if (infos[e].fault)
+      if (infos[e].fault == ADT_FAULT)
         return fail(ADT_EHIP, "batched: wave synchronisation timed out in event " + std::to_string(e));
   }
   if (probe)
@@ -2356,7 +2364,7 @@ int adt_graph_infos(adt_graph* g, adt_info* infos, void* stream) {
                          hipMemcpyDeviceToHost, s));
   ADT_HIP(hipStreamSynchronize(s));
   for (int e = 0; e < g->g->nev; ++e)
-    if (infos[e].fault)
+    if (infos[e].fault == ADT_FAULT)
       return fail(ADT_EHIP, "graph: wave synchronisation timed out in event " + std::to_string(e));
   return ADT_OK;
 }
@@ -2639,7 +2647,6 @@ int adt_selftest_forward(const adt_event3d* events, int32_t nev, int32_t flags, 
   if (nev < 1 || !forms || !left || (dtype != 0 && dtype != 1) ||
       (form != -1 && (form < ADT_FORM_ONE || form > ADT_FORM_WIDE)))
     return fail(ADT_EINVAL, "selftest: bad arguments");
-  for (int e = 0; e < nev; ++e) left[e] = 0;
   const ForwardProbe p{form, forms, left, infos == nullptr};
   return dtype == 0 ? batched_impl<double>(events, nev, flags, infos, stream, nullptr, &p)
                     : batched_impl<float>(events, nev, flags, infos, stream, nullptr, &p);

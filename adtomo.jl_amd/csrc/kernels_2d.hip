@@ -363,7 +363,7 @@ __global__ void __launch_bounds__(1024) fwd2_band_kernel(Event2Desc ev, int max_
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    if (flag[1]) ev.info->fault = 1;
+    if (flag[1]) ev.info->fault = ADT_FAULT;
     ev.info->iterations = conv ? it + 1 : it;
     ev.info->converged = conv ? 1 : 0;
     ev.info->err = (double)err;

@@ -261,7 +261,7 @@ struct Patience {
 };
 
 __device__ __forceinline__ void give_up(const EventDesc& ev, words_t hdr) {
-  ev.info->fault = 1;
+  ev.info->fault = ADT_FAULT;
   st_dev(&hdr[kAdjOver], 2);
 }
 

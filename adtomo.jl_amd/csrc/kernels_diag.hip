@@ -981,8 +981,12 @@ __device__ __forceinline__ void fwd3_diag_event(const EventDesc& ev, int max_ite
   __shared__ unsigned long long last_nan;
   const int m = ev.m, n = ev.n, l = ev.l;
   if (!ev.fwd_diag) return;  // handled by the k-streaming kernel
-  // solved by the team kernel unless that one gave it up
-  if (ev.team_words && ev.team_words[kTeamAbort] == 0) return;
+  // solved by the team kernel unless that one gave it up (2: a wait ran out)
+  if (ev.team_words) {
+    const int why = ev.team_words[kTeamAbort];
+    if (why == 0) return;
+    if (why == 2 && threadIdx.x == 0) ev.info->fault = ADT_FAULT_SOLVED;
+  }
   const int64_t N = (int64_t)m * n * l;
   const uint64_t bytes = (uint64_t)N * sizeof(T);
   if (threadIdx.x < 2) flags[threadIdx.x] = 0;
@@ -1095,7 +1099,7 @@ __device__ __forceinline__ void fwd3_diag_event(const EventDesc& ev, int max_ite
     ev.info->iterations = it > max_iter ? max_iter : it;
     ev.info->converged = (err < tol) ? 1 : 0;
     ev.info->err = (double)err;
-    if (flags[0]) ev.info->fault = 1;
+    if (flags[0]) ev.info->fault = ADT_FAULT;
   }
 }
 

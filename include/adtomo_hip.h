@@ -55,6 +55,10 @@ extern "C" {
 
 #define ADT_MAX_LOGGED_ITERS 100
 
+/* adt_info.fault */
+#define ADT_FAULT 1
+#define ADT_FAULT_SOLVED 2
+
 /* Per-call (per-event) diagnostics.  Replaces the reference's printf:
  * "ERROR: Eikonal does not converge!" (Eikonal.h:88-90) becomes
  * converged == 0; "Iteration %d, Error = %0.6e" (Eikonal3D.cpp:82-84)
@@ -68,8 +72,10 @@ typedef struct adt_info {
   int32_t ambiguous;     /* 2D: err within 1e-12 (rel) of the 1e-8 threshold */
   int32_t adj_sweeps;    /* adjoint Gauss-Seidel sweeps run */
   int32_t adj_converged; /* 1 if the adjoint reached its exact fixed point */
-  int32_t fault;         /* nonzero: a kernel's bounded wait for another wave
-                            timed out, so this event's results are invalid */
+  int32_t fault;         /* ADT_FAULT: a kernel's bounded wait for another wave
+                            timed out, so this event's results are invalid;
+                            ADT_FAULT_SOLVED: such a wait of the forward did, and
+                            another kernel then solved the event (valid, but late) */
   int64_t n_singular;    /* 2D adjoint: non-source nodes with no upwind
                             neighbour (singular rows in the reference) */
   double err_log[ADT_MAX_LOGGED_ITERS];
@@ -415,9 +421,10 @@ int adt_selftest_arith_f32(int32_t op, const float *a, const float *b, float *ou
  * As adt_eikonal3d_batched_* with the same events and flags, but with `form`
  * (ADT_FORM_ONE, _TEAM or _WIDE) in place of the library's choice where the
  * settings leave it open, or the library's (-1).  forms[nev]: what ran;
- * left[nev]: 0, or why several workgroups left the event to one (1: values
- * that their local solve does not cover, 2: a wait ran out).  With infos NULL
- * only the choice is made: nothing runs and no device is needed. */
+ * left[nev], out: 0, or why several workgroups left the event to one (1: values
+ * that their local solve does not cover, 2: a wait ran out); in: nonzero, and they
+ * leave it at once, as if for that reason.  With infos NULL only the choice is
+ * made: nothing runs and no device is needed. */
 #define ADT_FORM_STREAM 0 /* one workgroup, k-streaming */
 #define ADT_FORM_ONE 1    /* one workgroup, diagonals */
 #define ADT_FORM_TEAM 2   /* several workgroups, 16 bytes of k per lane */
