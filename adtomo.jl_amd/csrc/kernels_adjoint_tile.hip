@@ -46,12 +46,13 @@
 //
 // What bounds it.  One event: the chain of tiles along the rays, for each a load
 // (5000 cycles), some 25 rounds of 900 cycles (LDS reads, six products in order,
-// a division) and the hand-over (4000).  Many events: memory (256 events of
-// 128x128x64 read and write 58 GB in 9.5 ms), with two waves a SIMD to hide its
-// latency (LDS holds no more).  Measured,
+// a division) and the hand-over (4000).  Many events: memory (the tiles of 256
+// events of 128x128x64 read and write 34.7 GB in 7.6 ms, all three kernels 50.7 in
+// 10.8), with two waves a SIMD to hide its latency (LDS holds no more).  Measured,
 // prepare and solve, against one workgroup per event with its scheduling in LDS:
 // 128x128x64 FP64 12.7 -> 1.8 ms, 200x200x80 43 -> 4 ms, 400x400x160 460 -> 21 ms;
-// 64 events of 128x128x64 FP32 14.6 -> 4.5 ms; 256 of them FP64 17.1 -> 12.7 ms.
+// 64 events of 128x128x64 FP32 14.6 -> 4.5 ms; 256 of them FP64, 30 to 120 sources
+// each, 17.1 -> 12.7 ms (the benchmark's, 60 each, 10.8).
 #include "adjoint3.hpp"
 #include "buffer_ops.hpp"
 #include "eikonal_device.hpp"

@@ -52,17 +52,22 @@
 // then 32 nodes), whose memory accesses cover whole 64-byte columns and change
 // hands between lanes in LDS, one step ahead.  Its steps are 2.3 times as long, so
 // an event alone takes twice the time, but the accesses cost a fifth, and what
-// bounds it is the local solves (0.72 us per wave step and CU, two waves a SIMD:
-// its registers allow no third, and one with spills is slower).
+// bounds it is the local solves (0.6 us per wave step and CU, two waves a SIMD: the
+// 223 registers of FP64 allow no third, and one with spills is slower; the 152 of
+// FP32 and 167 with FP64 solves would, which was not tried).
 //
-// Measured, forward alone, one workgroup per event -> 16 bytes -> eight nodes, ms:
-// 128x128x64 FP64 28.3, 5.5, 10; 64x64x32 9.5, 1.8, 4.5; 16 events of 400x400x160
-// with FP32 storage 1476, 196, 106; 64 of 128x128x64 with FP32 storage 27.6, 17.9,
-// 12.2; 200 of 200x200x80 FP64 241, 347, 141; 256 of 128x128x64 FP64 48, 136, 49.
+// Measured, forward alone, one workgroup per event -> 16 bytes -> eight nodes, ms of
+// 20 iterations: 128x128x64 FP64 185, 37, 63; 64x64x32 94, 12, 30; 64 events of
+// 128x128x64 with FP32 storage 180, 112, 78; 200 of 200x200x80 FP64 1237, 2196, 878;
+// 256 of 128x128x64 FP64 250, 897, 297.  16 events of 400x400x160 with FP32 storage,
+// up to their stop rule, 1476, 196, 106.
 //
 // Values the fast local solve does not cover (NaN, -0, infinities, values of
 // 2^240 and more, discriminants below 2^-767) set the event's abort word; the
-// diagonal kernel launched behind this one then solves the event from u0.
+// diagonal kernel launched behind this one then solves the event from u0.  Such an
+// event costs more than with that kernel alone: its first sweep here (256 uneven
+// events with u0 infinite 52.0 -> 53.1 ms), and, where it is the only one of many, a
+// solve behind the others' (46.8 -> 67.4 ms).
 #include <type_traits>
 
 #include "buffer_ops.hpp"
