@@ -369,6 +369,12 @@ def _event_table(u0s, fs, hs, tols, grad_us, us, grad_u0s, grad_fs):
         elif f.dtype != dtype:
             raise ValueError("all events must share one dtype")
         m, n, l = f.shape
+        # the kernels take the box from f: nothing shorter may stand beside it
+        for name, x in (("u0", u0s), ("u", us), ("grad_u", grad_us), ("grad_u0", grad_u0s),
+                        ("grad_f", grad_fs)):
+            if x is not None and x[e].nbytes < f.nbytes:
+                raise ValueError(f"event {e}: {name} {tuple(x[e].shape)} ({x[e].dtype}) is smaller "
+                                 f"than f {tuple(f.shape)} ({f.dtype})")
         ev = tab[e]
         ev.m, ev.n, ev.l = m, n, l
         ev.h = float(hs[e])
