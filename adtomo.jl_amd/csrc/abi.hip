@@ -13,6 +13,7 @@
 #include <list>
 #include <map>
 #include <mutex>
+#include <numeric>
 #include <queue>
 #include <set>
 #include <string>
@@ -501,7 +502,10 @@ struct TeamPlan {
 };
 
 // The forms' times for one iteration, in microseconds as measured on an MI355X
-// with 20 iterations of every event (80 sets of events in each precision).
+// with 20 iterations of every event (some 110 sets of events in each precision).
+
+// The part of an array's columns of l nodes that do not begin on a multiple of w.
+double askew(int l, int w) { return 1 - (double)std::gcd(l, w) / w; }
 
 // One workgroup, an event alone: its steps, in chains of sweeps where all of k is
 // one chunk (20 us to begin a chain), 4.3 us a step with eight nodes a lane (FP32
@@ -522,8 +526,8 @@ double one_workgroup_us(const adt::EventDesc& d) {
   return us;
 }
 // One workgroup each: handed out largest first, or, where that is more, their
-// accesses: 64 bytes of u, f and u again for eight nodes (in FP32 as well), 1.6 times
-// as many where columns do not begin on them, at the rate of a large copy.
+// accesses: 64 bytes of u, f and u again for eight nodes (in FP32 as well), or twice
+// that for those that do not begin on eight, at the rate of a large copy.
 template <typename T>
 double one_workgroup_each_us(const std::vector<adt::EventDesc>& descs, int cus) {
   std::vector<double> us;
@@ -531,7 +535,7 @@ double one_workgroup_each_us(const std::vector<adt::EventDesc>& descs, int cus) 
   for (const adt::EventDesc& d : descs) {
     if (!d.fwd_diag) continue;
     us.push_back(one_workgroup_us<T>(d));
-    mem += 8 * 3 * 8.0 * d.m * d.n * d.l * (d.l % 8 ? 1.6 : 1) / 4.92e6;
+    mem += 8 * 3 * 8.0 * d.m * d.n * d.l * (1 + askew(d.l, 8)) / 4.92e6;
   }
   std::sort(us.begin(), us.end(), std::greater<double>());
   std::priority_queue<double, std::vector<double>, std::greater<double>> ends;
@@ -549,12 +553,13 @@ double one_workgroup_each_us(const std::vector<adt::EventDesc>& descs, int cus) 
 // Which forward kernel suits these events?  Several workgroups: an event alone
 // takes 4 (M_a + N_b) + 30 slabs + 80 steps (its sweeps overlap), many are bound by
 // the wave steps of all of them, on the CUs of the XCDs that have an event.  With
-// 16 bytes of k per lane 1.1 us a step and 0.44 us per CU for each wave step
-// (accesses to the L2, 16 bytes each); with eight nodes 2.6 us and 0.36 us + 0.40
-// for a step's worth of nodes (the local solves; 0.875 of it in FP32, 1.25 where
-// columns do not begin on 64 bytes), and more where the groups do not fill the
-// XCD: an event has slots / (events of an XCD) workgroups, rounded down, each
-// faster by a third of what the others leave idle.
+// 16 bytes of k per lane 1.1 us a step, and per CU 0.08 us for each wave step and 0.56
+// for 64 columns of it (accesses to the L2, 16 bytes each; 1.17 times that where they
+// do not begin on 16 bytes).  With eight nodes 2.6 us, 0.26 and 0.55 (the local
+// solves, and the columns' 64 bytes: 1.67 times where they do not begin on them, in
+// FP32 1.5), 0.92 of both in FP32, 0.3 of it for a wave of the slab that has no nodes; and more
+// where the groups do not fill the XCD: an event has slots / (events of an XCD)
+// workgroups, rounded down, each faster by a third of what the others leave idle.
 // How many iterations there are differs by event (2 and 3, or 3 and 4): one
 // workgroup each takes as long as the event with the most, the others as the mean.
 // So several workgroups are taken up to 1.05 times the first form's time.
@@ -583,10 +588,13 @@ Forward choose_forward(const std::vector<adt::EventDesc>& descs, const std::vect
     for (int w = 0; w < 2; ++w) {
       const adt::TeamDesc t = TeamPlan::geometry<T>(d, w == 1);
       const double segs = std::ceil(d.l / (w ? 8.0 : 16.0 / sizeof(T))), steps = Nb + t.H - 1;
-      const double wide = (0.36 * steps + 0.40 * Nb * t.H / 64) * (sizeof(T) == 8 ? 1 : 0.875) *
-                          (d.l % 8 ? 1.25 : 1);
+      const double cols = Nb * t.H / 64;
+      const double odd = sizeof(T) == 8 ? 0.67 : 0.5;
+      const double cost = w ? (0.26 * steps + 0.55 * cols * (1 + odd * askew(d.l, 8))) *
+                                  (sizeof(T) == 8 ? 1 : 0.92) * (0.7 + 0.3 * adt::kTW * t.ns / segs)
+                            : 0.08 * steps + 0.56 * cols * (1 + 0.17 * askew(d.l, 16 / sizeof(T)));
       tmax[w] = std::max(tmax[w], (4 * (Ma + Nb) + 30 * t.ns + 80) * (w ? 2.6 : 1.1));
-      tsum[w] += 8 * t.bands * segs * (w ? wide : 0.44 * steps);
+      tsum[w] += 8 * t.bands * segs * cost;
       if (w) maxR = std::max<int64_t>(maxR, t.R);
     }
   }
@@ -596,7 +604,7 @@ Forward choose_forward(const std::vector<adt::EventDesc>& descs, const std::vect
   const double td = one_workgroup_each_us<T>(descs, cus);
   const double t0 = std::max(tmax[0], tsum[0] / used), t1 = std::max(tmax[1], tsum[1] / used * idle);
   if (std::min(t0, t1) + one_workgroup_each_us<T>(rest, cus) >= 1.05 * td) return Forward::kOne;
-  return t0 <= t1 ? Forward::kTeam : Forward::kWide;
+  return 1.03 * t0 <= t1 ? Forward::kTeam : Forward::kWide;
 }
 
 void launch_clear(adt_info* infos, int nev, void* words, size_t bytes, hipStream_t s) {

@@ -28,6 +28,18 @@ def test_equal_boxes_of_one_band():
         assert forms([box] * 250, MODES[0]) == {"one"}
 
 
+def test_equal_boxes_of_odd_columns():
+    f64, mixed = MODES[0], MODES[2]
+    for box, n in [((93, 95, 59), 206), ((90, 120, 57), 200), ((126, 126, 64), 200)]:
+        assert forms([box] * n, f64) == {"one"}, (box, n)
+    for box, n in [((48, 33, 57), 247), ((40, 60, 63), 256), ((33, 160, 60), 256),
+                   ((76, 110, 61), 171), ((64, 64, 61), 200), ((50, 50, 64), 256)]:
+        assert forms([box] * n, f64) == {"wide"}, (box, n)
+    assert forms([(14, 160, 9)] * 338, mixed) == {"team"}
+    assert forms([(86, 93, 62)] * 213, mixed) == {"wide"}
+    assert forms([(24, 20, 12)] * 400, f64) == {"team"}
+
+
 @pytest.mark.parametrize("mode", MODES, ids=["f64", "f32", "mixed"])
 def test_boxes_that_stay_on_several_workgroups(mode):
     for box, n in [((200, 200, 80), 200), ((101, 90, 47), 256), ((96, 100, 48), 224),
